@@ -163,17 +163,17 @@ struct fxg_ctx {
   long long spec_elems = 0;
   // plain X
   std::vector<DevProd> prods;
-  DevProd* d_prods = nullptr;
-  // blocked plain X-engine: groups of rows, their pair tables and work items; the products it
-  // does not take (rows of groups above 64, repeated row pairs) stay with the per-product kernel
+  // matrix plain X-engine: groups of rows and work items, one run of items per row class; the
+  // products it does not take (groups above 64 rows or of mixed FFT stride, repeated row pairs)
+  // stay with the per-product kernel
   std::vector<XPGroup> xp_groups;
-  std::vector<XPRow> xp_rows;
-  std::vector<int> xp_pairs;
+  std::vector<long long> xp_rows;
   std::vector<XPItem> xp_items;
+  struct XPClass { int R, item0, nitems; };
+  std::vector<XPClass> xp_classes;
   std::vector<DevProd> prods_rest;
   XPGroup* d_xp_groups = nullptr;
-  XPRow* d_xp_rows = nullptr;
-  int* d_xp_pairs = nullptr;
+  long long* d_xp_rows = nullptr;
   XPItem* d_xp_items = nullptr;
   DevProd* d_prods_rest = nullptr;
   float2* d_xacc = nullptr;
@@ -184,18 +184,21 @@ struct fxg_ctx {
   std::vector<std::vector<std::pair<int, int>>> group_rows;   // (ds, band) per row
   std::map<std::pair<int, int>, std::pair<int, int>> rowof;   // (ds, recband) -> (group, row)
   DevXGroup* d_groups = nullptr;
+  // raw accumulator tiles of either X-engine and their reduction to product accumulators
   float* d_vacc = nullptr;
-  long long vacc_len = 0;
+  std::vector<XRGroup> xr_groups;
+  std::vector<long long> xr_pairs;
+  XRGroup* d_xr_groups = nullptr;
+  long long* d_xr_pairs = nullptr;
+  int xr_maxC = 0, xr_maxtp = 0;
   float* d_xscale = nullptr;
   long long xscale_len = 0;
   // accumulation entries
-  std::vector<FinPlain> finp;
-  std::vector<FinMfma> finm;
+  std::vector<FinProd> finp;
   std::vector<FinWeight> finw;
-  FinPlain* d_finp = nullptr;
-  FinMfma* d_finm = nullptr;
+  FinProd* d_finp = nullptr;
   FinWeight* d_finw = nullptr;
-  int maxoutp = 0, maxoutm = 0;
+  int maxoutp = 0;
   // amplitude scaling (Visibility::writedata)
   std::vector<NormSeg> normseg;
   std::vector<NormCal> normcal;     // + one zero entry at the end (bands without a mean)
@@ -1019,16 +1022,22 @@ int tile_width_log(const DevXGroup& g, int want) {
   return (want == 4 && g.ntile == 1 && g.C % 16 == 0) ? 4 : 3;
 }
 
-// The blocked plain X-engine's tables.  A row is a spectra band or zoom window with its channel
+// Splits of the X-engine's FFT loop: enough workgroups for the device where the channel tiles
+// alone (`units` workgroups) are too few, at least 16 FFTs each.
+int x_splits(const fxg_ctx* ctx, long long units, long long wanted) {
+  const long long most = std::max(1LL, (long long)std::min(ctx->chunkcap, ctx->B) / 16);
+  return (int)std::max(1LL, std::min(most, wanted / std::max(1LL, units)));
+}
+
+// The matrix plain X-engine's tables.  A row is a spectra band or zoom window with its channel
 // count, (datastream, band, channel offset, channels); products join rows into groups.  Each
 // group of at most 64 rows gets a pair table (the accumulator of the product of rows (i, j), or
-// -1) and work items of 8 x 8 row blocks over 64-channel tiles.  Products of groups above 64
-// rows or whose rows' datastreams differ in FFT stride, a second product of the same row pair,
-// and every product when the FP32 spectra reach 4 GiB (the kernel's offsets are 32-bit) stay
-// with the per-product kernel.
-void build_xplain_blocks(fxg_ctx* ctx) {
+// -1) and work items of XP_CT channels.  Products of groups above 64 rows or whose rows'
+// datastreams differ in FFT stride, and a second product of the same row pair, stay with the
+// per-product kernel.  Returns the floats of raw accumulator tiles.
+long long build_xplain(fxg_ctx* ctx) {
   const auto& P = ctx->prods;
-  ctx->xp_groups.clear(); ctx->xp_rows.clear(); ctx->xp_pairs.clear(); ctx->xp_items.clear();
+  ctx->xp_groups.clear(); ctx->xp_rows.clear(); ctx->xp_items.clear(); ctx->xp_classes.clear();
   ctx->prods_rest.clear();
   std::map<std::array<int, 4>, int> rid;
   std::vector<std::array<int, 4>> rkey;
@@ -1062,70 +1071,71 @@ void build_xplain_blocks(fxg_ctx* ctx) {
     local[r] = (int)grows[gid[g]].size();
     grows[gid[g]].push_back((int)r);
   }
-  if (8LL * ctx->spec_elems >= (1LL << 32)) {
-    ctx->prods_rest = P;
-    return;
-  }
   std::vector<int> gslot(grows.size(), -1);
   for (size_t g = 0; g < grows.size(); ++g) {
     const int n = (int)grows[g].size();
-    if (n > 64) continue;
+    if (n > XP_MAXROWS) continue;
     bool onestride = true;
     for (int r : grows[g]) onestride = onestride && ctx->h_ds[rkey[r][0]].C == ctx->h_ds[rkey[grows[g][0]][0]].C;
     if (!onestride) continue;
     XPGroup G;
+    std::memset(&G, 0, sizeof(G));
     G.nrows = n;
     G.C = rkey[grows[g][0]][3];
     G.stride = ctx->h_ds[rkey[grows[g][0]][0]].C;
-    G.pad = 0;
     G.row0 = (int)ctx->xp_rows.size();
-    G.pair0 = (int)ctx->xp_pairs.size();
     for (int r : grows[g]) {
       const DevDs& x = ctx->h_ds[rkey[r][0]];
-      XPRow R;
-      R.off = x.spec_off + (long long)rkey[r][1] * ctx->chunkcap * x.C + rkey[r][2];
-      R.stride = x.C;
-      R.pad = 0;
-      ctx->xp_rows.push_back(R);
+      ctx->xp_rows.push_back(x.spec_off + (long long)rkey[r][1] * ctx->chunkcap * x.C + rkey[r][2]);
     }
-    ctx->xp_pairs.resize(ctx->xp_pairs.size() + (size_t)n * n, -1);
+    XRGroup X;
+    std::memset(&X, 0, sizeof(X));
+    X.kind = n <= 16 ? XR_S16 : XR_S32;
+    X.n = n;
+    X.C = G.C;
+    X.ntile = n <= 32 ? 1 : 2;
+    X.pair0 = (int)ctx->xr_pairs.size();
+    ctx->xr_pairs.resize(ctx->xr_pairs.size() + (size_t)n * n, -1);
     gslot[g] = (int)ctx->xp_groups.size();
     ctx->xp_groups.push_back(G);
+    ctx->xr_groups.push_back(X);
   }
   for (size_t i = 0; i < P.size(); ++i) {
     const int gs = gslot[gid[root(r1[i])]];
     if (gs < 0) { ctx->prods_rest.push_back(P[i]); continue; }
-    const XPGroup& G = ctx->xp_groups[gs];
-    int& slot = ctx->xp_pairs[G.pair0 + (size_t)local[r1[i]] * G.nrows + local[r2[i]]];
+    const XRGroup& G = ctx->xr_groups[gs];
+    long long& slot = ctx->xr_pairs[G.pair0 + (size_t)local[r1[i]] * G.n + local[r2[i]]];
     if (slot >= 0) { ctx->prods_rest.push_back(P[i]); continue; }
     slot = P[i].acc_off;
   }
-  // Workgroups are dispatched to the eight XCDs in turn by workgroup index, and each XCD has
-  // its own L2: the blocks of one (group, channel tile), which read the same rows, go to one
-  // XCD (unit u to XCD u mod 8, its blocks at indices x, x + 8, ...); the shorter XCD lists
-  // are padded with empty items (group -1).
-  constexpr int NXCD = 8;
-  std::vector<std::vector<XPItem>> per(NXCD);
-  int unit = 0;
-  for (size_t gi = 0; gi < ctx->xp_groups.size(); ++gi) {
-    const XPGroup& G = ctx->xp_groups[gi];
-    const int nbk = (G.nrows + 7) / 8;
-    for (int c0 = 0; c0 < G.C; c0 += 64, ++unit)
-      for (int rb = 0; rb < nbk; ++rb)
-        for (int cb = rb; cb < nbk; ++cb) {
-          XPItem it;
-          it.group = (int)gi; it.rb = rb; it.cb = cb; it.c0 = c0;
-          per[unit % NXCD].push_back(it);
-        }
-  }
-  size_t len = 0;
-  for (const auto& v : per) len = std::max(len, v.size());
-  for (size_t k = 0; k < len; ++k)
-    for (int x = 0; x < NXCD; ++x) {
-      XPItem it;
-      it.group = -1; it.rb = 0; it.cb = 0; it.c0 = 0;
-      ctx->xp_items.push_back(k < per[x].size() ? per[x][k] : it);
+  // one launch per row class (16, 32 or 64 rows), split over the FFTs to fill the device: with
+  // four stations of one band (16 channel tiles, 125000 FFTs) one workgroup per tile took
+  // 30.5 ms
+  long long off = 0;
+  for (int R : {16, 32, 64}) {
+    auto cls = [&](const XPGroup& G) { return G.nrows <= 16 ? 16 : G.nrows <= 32 ? 32 : 64; };
+    long long units = 0;
+    for (const auto& G : ctx->xp_groups) if (cls(G) == R) units += (G.C + XP_CT - 1) / XP_CT;
+    if (!units) continue;
+    const int ns = x_splits(ctx, units, 4LL * ctx->ncu);
+    const int item0 = (int)ctx->xp_items.size();
+    for (size_t gi = 0; gi < ctx->xp_groups.size(); ++gi) {
+      XPGroup& G = ctx->xp_groups[gi];
+      if (cls(G) != R) continue;
+      G.off = off;
+      G.split_stride = (long long)G.C * R * R;
+      G.nsplit = ns;
+      off += ns * G.split_stride;
+      XRGroup& X = ctx->xr_groups[gi];
+      X.off = G.off;
+      X.split_stride = G.split_stride;
+      X.nsplit = ns;
+      for (int q = 0; q < ns; ++q)
+        for (int c0 = 0; c0 < G.C; c0 += XP_CT) ctx->xp_items.push_back(XPItem{(int)gi, c0, q});
     }
+    ctx->xp_classes.push_back({R, item0, (int)ctx->xp_items.size() - item0});
+  }
+  return off;
 }
 
 int build_engines(fxg_ctx* ctx, int chunk_req) {
@@ -1216,7 +1226,6 @@ int build_engines(fxg_ctx* ctx, int chunk_req) {
   } else {
     for (int d = 0; d < nds; ++d) per_fft += (long long)ctx->h_ds[d].nrecbands * ctx->h_ds[d].C * 8;
   }
-  // (FP32 spectra stay below 4 GiB: the blocked plain X-engine addresses them with 32-bit offsets)
   const long long budget = mfma ? (4LL << 30) : (4LL << 30) - (256LL << 20);
   long long cap = chunk_req > 0 ? chunk_req : std::max<long long>(64, budget / std::max<long long>(per_fft, 1));
   cap = std::min<long long>(cap, round_up(ctx->B, FXG_XPAD));
@@ -1229,13 +1238,14 @@ int build_engines(fxg_ctx* ctx, int chunk_req) {
       g.spec_off = off;
       g.rowstride = cap * g.C + 32;       // one 128-byte line of padding per row
       off += (long long)g.ntile * 32 * g.rowstride;
+      g.split_stride = (long long)g.C * (g.ntile * (g.ntile + 1) / 2) * 2 * 1024;
+      g.nsplit = 1;
       g.acc_off = aoff;
-      aoff += (long long)g.C * (g.ntile * (g.ntile + 1) / 2) * 2 * 1024;
+      aoff += g.nsplit * g.split_stride;
       g.scale_off = soff;
       soff += (long long)g.ntile * 32;                 // one scale per input row
     }
     ctx->spec_elems = off;
-    ctx->vacc_len = aoff;
     ctx->xscale_len = soff;
     if (int rc_ = dev_malloc(ctx, (void**)&ctx->d_spec16, sizeof(uint32_t) * std::max<long long>(off, 4))) return rc_;
     if (int rc_ = dev_zero(ctx, ctx->d_spec16, sizeof(uint32_t) * std::max<long long>(off, 4))) return rc_;
@@ -1275,11 +1285,11 @@ int build_engines(fxg_ctx* ctx, int chunk_req) {
       p.ds1 = d1; p.band1 = b1; p.choff1 = c1;
       p.ds2 = d2; p.band2 = b2; p.choff2 = c2;
       p.nchan = nchan;
-      p.acc_off = (int)acc;
+      p.acc_off = acc;
       acc += nchan;
       ctx->prods.push_back(p);
       ctx->maxchan = std::max(ctx->maxchan, nchan);
-      return (long long)p.acc_off;
+      return p.acc_off;
     };
     for (int j = 0; j < nb; ++j) {
       const fxg_baseline& b = ctx->bls[j];
@@ -1292,7 +1302,7 @@ int build_engines(fxg_ctx* ctx, int chunk_req) {
           band_source(ctx->dss[b.ds1], b.ds1band[k][p], &r1, &c1);
           band_source(ctx->dss[b.ds2], b.ds2band[k][p], &r2, &c2);
           long long src = add_prod(b.ds1, r1, c1, b.ds2, r2, c2, fr.nchan);
-          FinPlain e;
+          FinProd e;
           e.src = src;
           e.dst = ctx->boff[(size_t)f * nb + j] + p * nout;
           e.nout = nout;
@@ -1328,7 +1338,7 @@ int build_engines(fxg_ctx* ctx, int chunk_req) {
           band_source(s, b, &rec, &choff);
           long long src = w == 0 ? aacc[rec] : xacc[rec];
           if (src >= 0) {
-            FinPlain e;
+            FinProd e;
             e.src = src + choff;
             e.dst = (int)idx;
             e.nout = nout;
@@ -1345,18 +1355,40 @@ int build_engines(fxg_ctx* ctx, int chunk_req) {
     }
     ctx->xacc_len = acc;
     if (int rc_ = dev_malloc(ctx, (void**)&ctx->d_xacc, sizeof(float2) * std::max<long long>(acc, 2))) return rc_;
-    if (int rc = dev_upload(ctx, &ctx->d_prods, ctx->prods)) return rc;
-    if (int rc = dev_upload(ctx, &ctx->d_finp, ctx->finp)) return rc;
-    build_xplain_blocks(ctx);
+    const long long plen = build_xplain(ctx);
     if (!ctx->xp_items.empty()) {
+      if (int rc = dev_malloc(ctx, (void**)&ctx->d_vacc, (long long)sizeof(float) * plen)) return rc;
       if (int rc = dev_upload(ctx, &ctx->d_xp_groups, ctx->xp_groups)) return rc;
       if (int rc = dev_upload(ctx, &ctx->d_xp_rows, ctx->xp_rows)) return rc;
-      if (int rc = dev_upload(ctx, &ctx->d_xp_pairs, ctx->xp_pairs)) return rc;
       if (int rc = dev_upload(ctx, &ctx->d_xp_items, ctx->xp_items)) return rc;
     }
     if (!ctx->prods_rest.empty())
       if (int rc = dev_upload(ctx, &ctx->d_prods_rest, ctx->prods_rest)) return rc;
   } else {
+    // a pair table per group: the accumulator of each ordered row pair that a product uses
+    for (size_t g = 0; g < ctx->groups.size(); ++g) {
+      const DevXGroup& G = ctx->groups[g];
+      XRGroup X;
+      std::memset(&X, 0, sizeof(X));
+      X.kind = XR_H;
+      X.n = G.nin;
+      X.C = G.C;
+      X.ntile = G.ntile;
+      X.off = G.acc_off;
+      X.split_stride = G.split_stride;
+      X.nsplit = G.nsplit;
+      X.scale_off = G.scale_off;
+      X.pair0 = (int)ctx->xr_pairs.size();
+      ctx->xr_pairs.resize(ctx->xr_pairs.size() + (size_t)G.nin * G.nin, -1);
+      ctx->xr_groups.push_back(X);
+    }
+    long long acc = 0;
+    auto pair_acc = [&](int g, int i, int j) {
+      const XRGroup& X = ctx->xr_groups[g];
+      long long& slot = ctx->xr_pairs[X.pair0 + (size_t)i * X.n + j];
+      if (slot < 0) { slot = acc; acc += X.C; }
+      return slot;
+    };
     for (int j = 0; j < nb; ++j) {
       const fxg_baseline& b = ctx->bls[j];
       for (int k = 0; k < b.nfreqs; ++k) {
@@ -1367,20 +1399,16 @@ int build_engines(fxg_ctx* ctx, int chunk_req) {
           auto g1 = ctx->rowof[{b.ds1, b.ds1band[k][p]}];
           auto g2 = ctx->rowof[{b.ds2, b.ds2band[k][p]}];
           if (g1.first != g2.first) return fail(ctx, FXG_E_INVALID, "product rows in different MFMA groups");
-          FinMfma e;
-          e.group = g1.first;
-          e.row1 = g1.second;
-          e.row2 = g2.second;
-          e.chan0 = 0;
+          FinProd e;
+          e.src = pair_acc(g1.first, g1.second, g2.second);
           e.dst = ctx->boff[(size_t)f * nb + j] + p * nout;
           e.nout = nout;
           e.avg = fr.chanavg;
-          e.isauto = 0;
           e.bl = j;
           e.fq = f;
           e.pcstride = b.npolprod[k] * nout;
-          ctx->finm.push_back(e);
-          ctx->maxoutm = std::max(ctx->maxoutm, nout);
+          ctx->finp.push_back(e);
+          ctx->maxoutp = std::max(ctx->maxoutp, nout);
         }
       }
     }
@@ -1402,27 +1430,59 @@ int build_engines(fxg_ctx* ctx, int chunk_req) {
           if (other >= 0) {
             auto g1 = ctx->rowof[{d, rec}];
             auto g2 = ctx->rowof[{d, other}];
-            FinMfma e;
-            e.group = g1.first;
-            e.row1 = g1.second;
-            e.row2 = g2.second;
-            e.chan0 = choff;
+            FinProd e;
+            e.src = pair_acc(g1.first, g1.second, g2.second) + choff;
             e.dst = (int)idx;
             e.nout = nout;
             e.avg = cavg;
-            e.isauto = (w == 0);
             e.bl = -1;
             e.fq = 0;
             e.pcstride = 0;
-            ctx->finm.push_back(e);
-            ctx->maxoutm = std::max(ctx->maxoutm, nout);
+            ctx->finp.push_back(e);
+            ctx->maxoutp = std::max(ctx->maxoutp, nout);
           }
           idx += nout;
         }
       }
     }
-    if (int rc = dev_upload(ctx, &ctx->d_finm, ctx->finm)) return rc;
+    ctx->xacc_len = acc;
+    if (int rc = dev_malloc(ctx, (void**)&ctx->d_xacc, (long long)sizeof(float2) * std::max<long long>(acc, 2))) return rc;
   }
+  // products that go to the results channel by channel (one phase centre, no averaging, no other
+  // reader such as a zoom window) are written there by the reduction itself
+  if (ctx->nphase <= 1) {
+    std::map<long long, std::pair<long long*, int>> slot;          // accumulator -> entry, channels
+    for (const auto& X : ctx->xr_groups)
+      for (int k = 0; k < X.n * X.n; ++k)
+        if (ctx->xr_pairs[X.pair0 + k] >= 0) slot[ctx->xr_pairs[X.pair0 + k]] = {&ctx->xr_pairs[X.pair0 + k], X.C};
+    std::map<long long, int> readers;
+    auto of = [&](long long src) {
+      auto it = slot.upper_bound(src);
+      if (it == slot.begin()) return slot.end();
+      --it;
+      return src < it->first + it->second.second ? it : slot.end();
+    };
+    for (const auto& e : ctx->finp) {
+      auto it = of(e.src);
+      if (it != slot.end()) readers[it->first]++;
+    }
+    std::vector<FinProd> rest;
+    for (const auto& e : ctx->finp) {
+      auto it = of(e.src);
+      if (it != slot.end() && it->first == e.src && readers[e.src] == 1 && e.avg == 1 && e.nout == it->second.second)
+        *it->second.first = -2 - (long long)e.dst;
+      else
+        rest.push_back(e);
+    }
+    ctx->finp.swap(rest);
+  }
+  for (const auto& X : ctx->xr_groups) {
+    ctx->xr_maxC = std::max(ctx->xr_maxC, X.C);
+    ctx->xr_maxtp = std::max(ctx->xr_maxtp, X.ntile * (X.ntile + 1) / 2);
+  }
+  if (int rc = dev_upload(ctx, &ctx->d_finp, ctx->finp)) return rc;
+  if (int rc = dev_upload(ctx, &ctx->d_xr_groups, ctx->xr_groups)) return rc;
+  if (int rc = dev_upload(ctx, &ctx->d_xr_pairs, ctx->xr_pairs)) return rc;
   // weights (core.cpp:1005-1052, 1306-1370)
   for (int f = 0; f < ctx->nfreqs; ++f) {
     if (!ctx->used[f]) continue;
@@ -1831,11 +1891,9 @@ int run_subint(fxg_ctx* ctx, const int32_t offsets[3], const uint8_t* const* d_d
 
   const bool mfma = ctx->xengine != FXG_X_FP32;
   if (fxg_launch_zero(d_results, ctx->coreresultlength * 8, st)) return fail(ctx, FXG_E_HIP, "zero results");
-  if (mfma) {
-    if (fxg_launch_zero(ctx->d_vacc, ctx->vacc_len * 4, st)) return fail(ctx, FXG_E_HIP, "zero acc");
-  } else {
-    if (fxg_launch_zero(ctx->d_xacc, ctx->xacc_len * 8, st)) return fail(ctx, FXG_E_HIP, "zero acc");
-  }
+  // (the per-product kernel adds to its accumulators; the others are overwritten)
+  if (!ctx->prods_rest.empty() && fxg_launch_zero(ctx->d_xacc, ctx->xacc_len * 8, st))
+    return fail(ctx, FXG_E_HIP, "zero acc");
   SetupArgs sa;
   sa.ds = ctx->d_ds;
   sa.run = ctx->d_run;
@@ -1908,16 +1966,19 @@ int run_subint(fxg_ctx* ctx, const int32_t offsets[3], const uint8_t* const* d_d
   UvArgs uv{nullptr, ctx->d_uvfreq, uvs ? ctx->nphase : 1};
   auto accumulate = [&](const UvArgs& u) -> int {
     TimedLaunch tl(ctx, 2, st);
-    if (mfma) {
-      if (fxg_launch_fin_mfma(ctx->d_finm, (int)ctx->finm.size(), ctx->maxoutm, ctx->d_groups, ctx->d_vacc,
-                              ctx->d_xscale, d_results, u, st))
-        return fail(ctx, FXG_E_HIP, "accumulate launch");
-    } else {
-      if (fxg_launch_fin_plain(ctx->d_finp, (int)ctx->finp.size(), ctx->maxoutp, ctx->d_xacc, d_results, u, st))
-        return fail(ctx, FXG_E_HIP, "accumulate launch");
-    }
+    XReduceArgs ra;
+    ra.groups = ctx->d_xr_groups;
+    ra.pairs = ctx->d_xr_pairs;
+    ra.part = ctx->d_vacc;
+    ra.xscale = ctx->d_xscale;
+    ra.acc = ctx->d_xacc;
+    ra.res = d_results;
+    if (fxg_launch_xreduce(ra, mfma, (int)ctx->xr_groups.size(), ctx->xr_maxC, ctx->xr_maxtp, st) ||
+        fxg_launch_fin(ctx->d_finp, (int)ctx->finp.size(), ctx->maxoutp, ctx->d_xacc, d_results, u, st))
+      return fail(ctx, FXG_E_HIP, "accumulate launch");
     return FXG_OK;
   };
+  int first = 1;                                   // the accumulators start here
   for (const auto& piece : pieces) {
     const int c0 = piece[0], n = piece[1];
     const int npad = (int)round_up(n, FXG_XPAD);
@@ -1943,6 +2004,7 @@ int run_subint(fxg_ctx* ctx, const int32_t offsets[3], const uint8_t* const* d_d
       xa.groups = ctx->d_groups;
       xa.spec16 = ctx->d_spec16;
       xa.acc = ctx->d_vacc;
+      xa.first = first;
       xa.nffts_pad = npad;
       xa.chunkcap = ctx->chunkcap;
       xa.mode = ctx->xengine;
@@ -1952,25 +2014,25 @@ int run_subint(fxg_ctx* ctx, const int32_t offsets[3], const uint8_t* const* d_d
       while (g0 < ctx->groups.size()) {
         size_t g1 = g0 + 1;
         while (g1 < ctx->groups.size() && ctx->groups[g1].ntile == ctx->groups[g0].ntile &&
-               ctx->groups[g1].C == ctx->groups[g0].C && ctx->groups[g1].twlog == ctx->groups[g0].twlog)
+               ctx->groups[g1].C == ctx->groups[g0].C && ctx->groups[g1].twlog == ctx->groups[g0].twlog &&
+               ctx->groups[g1].nsplit == ctx->groups[g0].nsplit)
           ++g1;
-        if (fxg_launch_xmfma(xa, (int)(g1 - g0), (int)g0, ctx->groups[g0].ntile, ctx->groups[g0].C,
-                             ctx->groups[g0].twlog, st))
+        if (fxg_launch_xmfma(xa, (int)(g1 - g0), (int)g0, ctx->groups[g0], st))
           return fail(ctx, FXG_E_HIP, "MFMA X-engine launch");
         g0 = g1;
       }
     } else {
       TimedLaunch tl(ctx, 1, st);
-      if (!ctx->xp_items.empty()) {
-        XPBlkArgs ba;
-        ba.items = ctx->d_xp_items;
-        ba.groups = ctx->d_xp_groups;
-        ba.rows = ctx->d_xp_rows;
-        ba.pairs = ctx->d_xp_pairs;
-        ba.spec32 = ctx->d_spec32;
-        ba.acc = ctx->d_xacc;
-        ba.nffts = n;
-        if (fxg_launch_xplain_blk(ba, (int)ctx->xp_items.size(), st)) return fail(ctx, FXG_E_HIP, "X-engine launch");
+      XPMatArgs ba;
+      ba.groups = ctx->d_xp_groups;
+      ba.rows = ctx->d_xp_rows;
+      ba.spec32 = ctx->d_spec32;
+      ba.part = ctx->d_vacc;
+      ba.nffts = n;
+      ba.first = first;
+      for (const auto& xc : ctx->xp_classes) {
+        ba.items = ctx->d_xp_items + xc.item0;
+        if (fxg_launch_xplain_mat(ba, xc.R, xc.nitems, st)) return fail(ctx, FXG_E_HIP, "X-engine launch");
       }
       if (!ctx->prods_rest.empty()) {
         XPlainArgs xa;
@@ -2002,10 +2064,12 @@ int run_subint(fxg_ctx* ctx, const int32_t offsets[3], const uint8_t* const* d_d
     }
     ctx->last_chunk0 = c0;
     ctx->last_nffts = n;
+    first = 0;
     if (piece[2] >= 0) {                           // end of a uv-shift interval
       uv.dd = sg.d_uvdd + (size_t)piece[2] * ctx->nbl * ctx->nphase;
       if (int rc = accumulate(uv)) return rc;
-      if (mfma ? fxg_launch_zero(ctx->d_vacc, ctx->vacc_len * 4, st) : fxg_launch_zero(ctx->d_xacc, ctx->xacc_len * 8, st))
+      first = 1;
+      if (!ctx->prods_rest.empty() && fxg_launch_zero(ctx->d_xacc, ctx->xacc_len * 8, st))
         return fail(ctx, FXG_E_HIP, "zero acc");
     }
   }
@@ -2150,9 +2214,9 @@ void free_ctx(fxg_ctx* ctx) {
   f(ctx->d_twiddle); f(ctx->d_dslist); f(ctx->d_params); f(ctx->d_items[0]); f(ctx->d_items[1]);
   f(ctx->d_iclass[0]); f(ctx->d_iclass[1]);
   f(ctx->d_counter); f(ctx->d_bigscratch); f(ctx->d_weights); f(ctx->d_flags); f(ctx->d_spec32); f(ctx->d_spec16);
-  f(ctx->d_prods); f(ctx->d_xp_groups); f(ctx->d_xp_rows); f(ctx->d_xp_pairs); f(ctx->d_xp_items);
+  f(ctx->d_xp_groups); f(ctx->d_xp_rows); f(ctx->d_xp_items); f(ctx->d_xr_groups); f(ctx->d_xr_pairs);
   f(ctx->d_prods_rest); f(ctx->d_xacc); f(ctx->d_groups); f(ctx->d_vacc); f(ctx->d_xscale);
-  f(ctx->d_finp); f(ctx->d_finm); f(ctx->d_finw);
+  f(ctx->d_finp); f(ctx->d_finw);
   f(ctx->d_normseg); f(ctx->d_normcal); f(ctx->d_calmean); f(ctx->d_tsys); f(ctx->d_dpct);
   f(ctx->d_kurt_tab); f(ctx->d_kurt_acc); f(ctx->d_pcal_groups); f(ctx->d_pcal_part); f(ctx->d_pcal_bins); f(ctx->d_pcal_tdev); f(ctx->d_pcal_tonebuf);
   f(ctx->d_uvfreq); f(ctx->d_uvdec_idx);

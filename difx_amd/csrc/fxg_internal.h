@@ -91,7 +91,7 @@ struct DevProd {
   int ds1, band1, choff1; // first operand: spectra band and channel offset (zoom windows)
   int ds2, band2, choff2; // second operand (conjugated)
   int nchan;              // channels of the product
-  int acc_off;            // cf32 offset of its accumulator
+  long long acc_off;      // cf32 offset of its accumulator
 };
 
 // MFMA X-engine group: one recorded frequency with its inputs (station bands).
@@ -105,7 +105,8 @@ struct DevXGroup {
   long long scale_off;    // float offset of its per-row scales [rows]
   int twlog;              // log2 of the channel tile width TW (8 or 16): spectra rows are
                           // [C/TW][t][TW] words, so one FFT writes TW channels contiguously
-  int pad_;
+  int nsplit;             // workgroups per channel tile, each a range of the chunk's FFTs
+  long long split_stride; // floats between the accumulators of its splits
 };
 
 // Frame flags of a slot buffer: 0 blanked, 1 every sample decodes, 2 only the time samples
@@ -214,36 +215,59 @@ struct XPlainArgs {
   int chunkcap;
 };
 
-// Blocked plain FP32 X-engine.  A group is a set of rows (spectra bands, or zoom windows of
-// them, with one channel count) that products connect; a work item is one 8 x 8 block (row
-// block rb <= column block cb) of the group's row x row matrix over 64 consecutive channels.
-struct XPRow {
-  long long off;          // cf32 offset in the FP32 spectra of (band, FFT 0, window start)
-  int stride;             // cf32 entries between consecutive FFTs
-  int pad;
-};
+// Plain FP32 X-engine on FP32 matrix instructions.  A group is a set of rows (spectra bands,
+// or zoom windows of them, with one channel count and FFT stride) that products connect; a work
+// item is XP_CT consecutive channels of one group.
+#define XP_CT 16            // channels per work item
+#define XP_MAXROWS 64       // rows per group (larger groups: per-product kernel)
 struct XPGroup {
-  int nrows, C, row0, pair0;   // pairs[pair0 + i*nrows + j]: accumulator of product (i, j) or -1
-  int stride;                  // cf32 entries between consecutive FFTs, the same for every row
-  int pad;
+  int nrows, C, row0;       // rows[row0 + i]: cf32 offset of (band, FFT 0, window start)
+  int stride;               // cf32 entries between consecutive FFTs, the same for every row
+  long long off;            // float offset of its accumulators: per channel the R x R matrix S
+  long long split_stride;   // floats between the accumulators of its splits
+  int nsplit, pad;
 };
 struct XPItem {
-  int group, rb, cb, c0;
+  int group, c0, split;     // split: which of the group's nsplit ranges of the chunk's FFTs
 };
-struct XPBlkArgs {
+struct XPMatArgs {
   const XPItem* items;
   const XPGroup* groups;
-  const XPRow* rows;
-  const int* pairs;
+  const long long* rows;
   const float2* spec32;
-  float2* acc;
+  float* part;              // raw accumulator tiles
   int nffts;
+  int first;                // 1: start from zero; 0: go on from the stored accumulators
+};
+
+// Raw accumulator tiles of either X-engine into per-product rows of channels: the splits over
+// FFTs are summed in order and product (i, j) of a group goes, by its pair table entry p, to
+// acc[p + c] (p >= 0), straight to the results, res[-2 - p + c] (p <= -2), or nowhere (-1).
+#define XR_S16 0            // FP32, one 16 x 16 tile S per channel
+#define XR_S32 1            // FP32, ntile^2 32 x 32 tiles S per channel
+#define XR_H 2              // 16-bit, (re, im) 32 x 32 tiles of the lower tile pairs per channel
+struct XRGroup {
+  int kind, n, C, ntile;
+  long long off;            // float offset of split 0, channel 0
+  long long split_stride;
+  long long scale_off;      // XR_H: float offset of its per-row scales
+  int pair0;                // first entry of its n x n pair table 
+  int nsplit;
+};
+struct XReduceArgs {
+  const XRGroup* groups;
+  const long long* pairs;
+  const float* part;
+  const float* xscale;
+  float2* acc;
+  float2* res;
 };
 
 struct XMfmaArgs {
   const DevXGroup* groups;
   const uint32_t* spec16;
   float* acc;
+  int first;              // 1: start from zero; 0: go on from the stored accumulators
   int nffts_pad;          // multiple of 8
   int chunkcap;
   int mode;               // 1 = FP16, 2 = BF16
@@ -270,7 +294,7 @@ struct UvArgs {
 };
 
 // Accumulation of a product accumulator into the results (core.cpp:1819-1853).
-struct FinPlain {
+struct FinProd {
   long long src;          // cf32 offset in the product accumulators
   int dst;                // cf32 offset in results (phase centre 0)
   int nout;               // output channels
@@ -278,17 +302,6 @@ struct FinPlain {
   int bl;                 // baseline of a cross product (-1: autocorrelation, not shifted)
   int fq;                 // freq of the product (uv-shift rotation constants)
   int pcstride;           // cf32 offset between the phase-centre blocks
-};
-
-struct FinMfma {
-  int group;
-  int row1, row2;         // V[row1][row2] (row1 is the unconjugated operand)
-  int chan0;              // first channel of the group spectrum (zoom window)
-  int dst;
-  int nout;
-  int avg;
-  int isauto;             // parallel-hand autocorrelation: imaginary part forced to zero
-  int bl, fq, pcstride;   // as FinPlain
 };
 
 struct FinWeight {
@@ -300,7 +313,8 @@ int fxg_launch_setup(const SetupArgs& a, int maxframes, hipStream_t st);
 int fxg_launch_unpack(const UnpackArgs& a, hipStream_t st);
 int fxg_launch_fengine(const FengineArgs& a, int L, int iscomplex, int nds, int ntb, hipStream_t st);
 int fxg_launch_fftparams(const FengineArgs& a, int nds, hipStream_t st);
-int fxg_launch_xplain_blk(const XPBlkArgs& a, int nitems, hipStream_t st);
+int fxg_launch_xplain_mat(const XPMatArgs& a, int R, int nitems, hipStream_t st);
+int fxg_launch_xreduce(const XReduceArgs& a, int mfma, int ngroups, int maxC, int maxtp, hipStream_t st);
 int fxg_launch_fpersist(const FengineArgs& a, const FItem* items, const IClass* cls, int ncls, int* counters,
                         int nwg, int ntb, int iscomplex, size_t lds, hipStream_t st);
 size_t fxg_fengine_lds(int L, int ntb, int phcap, int order);
@@ -308,11 +322,8 @@ int fxg_launch_fbig(const FengineArgs& a, int L, int iscomplex, int nds, int wgx
                     const float2* twL, hipStream_t st);
 size_t fxg_fbig_lds(int ntb, int phcap);
 int fxg_launch_xplain(const XPlainArgs& a, int nprod, int maxchan, hipStream_t st);
-int fxg_launch_xmfma(const XMfmaArgs& a, int ngroup_launch, int group0, int ntile, int C, int twlog, hipStream_t st);
-int fxg_launch_fin_plain(const FinPlain* e, int n, int maxout, const float2* acc, float2* res, const UvArgs& uv,
-                         hipStream_t st);
-int fxg_launch_fin_mfma(const FinMfma* e, int n, int maxout, const DevXGroup* g, const float* acc,
-                        const float* xscale, float2* res, const UvArgs& uv, hipStream_t st);
+int fxg_launch_xmfma(const XMfmaArgs& a, int ngroup_launch, int group0, const DevXGroup& g, hipStream_t st);
+int fxg_launch_fin(const FinProd* e, int n, int maxout, const float2* acc, float2* res, const UvArgs& uv, hipStream_t st);
 int fxg_launch_add_at(const int* idx, const float* val, int n, float* resf, hipStream_t st);
 int fxg_launch_fin_weights(const FinWeight* e, int n, const float* w, int B, float* resf, hipStream_t st);
 int fxg_launch_zero(void* p, long long bytes, hipStream_t st);

@@ -4,10 +4,9 @@
 //   acc += F1[t][c] * conj(F2[t][c])
 // over the FFTs of the subint in FP32, the vectorAddProduct_cf32 of Core::processdata
 // (mpifxcorr/src/core.cpp:884-979, :963) for the cross products and of Mode::process for the
-// autocorrelations (mode.cpp:1272, 1333-1339).  The blocked kernel takes 8 x 8 blocks of the
-// input x input matrix of the products' inputs (FFT order within each quarter of a chunk, the
-// quarters in order); the per-product kernel (one thread per product and channel, FFT order)
-// takes the products it leaves.
+// autocorrelations (mode.cpp:1272, 1333-1339).  The matrix kernel takes the input x input
+// matrix of the products' inputs per channel on FP32 matrix instructions; the per-product
+// kernel (one thread per product and channel, FFT order) takes the products it leaves.
 //
 // MFMA path: per channel the visibilities of all inputs (station bands of one frequency)
 // form the Hermitian matrix V = sum_t x_t x_t^H.  With x stored as interleaved (re, im)
@@ -57,113 +56,188 @@ __global__ void __launch_bounds__(256) k_xmac_f32(XPlainArgs a) {
 }
 
 
-// Blocked form of the plain FP32 X-engine: one workgroup per work item (an 8 x 8 block of a
-// group's row x row matrix over 64 channels, one channel per lane).  Each of the four
-// wavefronts sums X_i conj(X_j) over a quarter of the chunk's FFTs in FFT order, loading 16
-// spectra values per FFT for 64 products; wave 0 then adds the four partial sums in wave order
-// and adds the result to each product's accumulator: product (i, j) takes the block entry,
-// product (j, i) its conjugate (off the diagonal blocks).  Autocorrelations (i = j) keep a zero
-// imaginary part.  Rows past the group and channels past C are clamped for the loads and never
-// written.  Items with group -1 are padding and do nothing.
-__global__ void __launch_bounds__(256) k_xmac_f32_blk(XPBlkArgs a) {
-  __shared__ float2 red[3][16][64];
+// Matrix form of the plain FP32 X-engine.  Per channel and FFT the rows' spectra x give
+//   S = re(x) (re(x) - im(x))^T + im(x) (re(x) + im(x))^T,
+// one FP32 matrix product over k = (re, im), and V = x x^H follows from it:
+//   re V = (S + S^T) / 2,  im V = (S - S^T) / 2
+// (re V is symmetric and im V antisymmetric), so one FP32 matrix instruction per FFT does the
+// work of a real and an imaginary one.  Inputs, products and sums stay FP32.
+// A workgroup takes XP_CT channels of one group (one 128-byte line per row and FFT) and a range
+// of the chunk's FFTs; TB FFTs at a time are staged in LDS as [FFT][row][channel] (one pad entry
+// per row: a wave's reads, one row per lane, then hit distinct banks), double buffered, the next
+// stage's loads in flight while the current one is multiplied.  Rows past the group stay zero.
+// Runs of 256 FFTs (512 for R = 64) are summed apart and then added to the total: one chain over
+// 7800 FFTs of 10 stations was 1.3e-6 off the 64-bit result, against 1.8e-7 in quarters of a chunk.
+// R is the row count rounded up to 16, 32 or 64 (16x16x4 tiles, else 32x32x2).
+template <int R>
+struct XPTile {
+  static constexpr int NTH = 16 * R;                      // waves of 4, 2 or 1 channels: the accumulators
+                                                          // of a channel are 8, 32 or 64 registers
+  static constexpr int NW = NTH / 64;
+  static constexpr int CPW = XP_CT / NW;                  // channels per wave
+  static constexpr int TB = 128 / R;                      // FFTs per stage
+  static constexpr int RS = XP_CT + 1;                    // LDS entries per row
+  static constexpr int STAGE = TB * R * RS;
+  static constexpr int QN = TB * R * (XP_CT / 2) / NTH;   // 16-byte loads per thread and stage
+  static constexpr int NT = R == 64 ? 2 : 1;              // row tiles
+  static constexpr int RR = R * R;                        // accumulators per channel
+  static constexpr int RUN = (R == 64 ? 512 : 256) / TB;  // stages summed before they join the total
+};
+typedef float floatx4 __attribute__((ext_vector_type(4)));
+typedef float float4_a8 __attribute__((ext_vector_type(4), aligned(8)));
+
+template <int R>
+__global__ void __launch_bounds__(XPTile<R>::NTH) k_xmac_f32_mat(XPMatArgs a) {
+  using T = XPTile<R>;
+  constexpr int NT = T::NT, CPW = T::CPW, TB = T::TB, RS = T::RS, QN = T::QN;
+  constexpr int NREG = R == 16 ? 4 : 16;
+  __shared__ float2 lds[2][T::STAGE];
   const XPItem it = a.items[blockIdx.x];
-  if (it.group < 0) return;                      // padding item: the whole workgroup leaves
   const XPGroup g = a.groups[it.group];
-  const int lane = threadIdx.x & 63;
-  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);   // wave-uniform: scalar loop and pointers
-  const int c = it.c0 + lane;
-  const int cl = min(c, g.C - 1);
-  // the row pointers are the same for every lane (scalar registers); each lane adds its channel
-  const int t0 = (int)((long long)w * a.nffts / 4), t1 = (int)((long long)(w + 1) * a.nffts / 4);
-  // 32-bit byte offsets from the spectra base (the host keeps the FP32 spectra below 4 GiB
-  // for this kernel), so each load is the scalar base plus one offset register
-  typedef float v2f __attribute__((ext_vector_type(2)));
-  typedef const __attribute__((address_space(1))) v2f* GF2;
-  typedef const __attribute__((address_space(1))) char* GB;
-  // The rows of a group share one FFT stride, so the row offsets are the same for every lane
-  // (scalar registers) and each load adds the lane's channel offset.
-  const GB base = (GB)a.spec32;
-  unsigned ox[8], oy[8];
-  const unsigned st = 8u * (unsigned)g.stride;
-  const unsigned co = (unsigned)cl * 8u;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int t0 = (int)((long long)it.split * a.nffts / g.nsplit);
+  const int t1 = (int)((long long)(it.split + 1) * a.nffts / g.nsplit);
+  const int nc = g.C - it.c0;                             // channels left (the last item may be short)
+
+  for (int i = tid; i < 2 * T::STAGE; i += T::NTH) (&lds[0][0])[i] = make_float2(0.0f, 0.0f);
+
+  // load q of a stage: FFT q / (8 R), row (q / 8) % R, channels 2 (q % 8) and the next
+  const float2* src[QN];
+  bool on[QN];
+  int tq[QN], dst[QN];
 #pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    ox[i] = (unsigned)(8LL * (a.rows[g.row0 + min(it.rb * 8 + i, g.nrows - 1)].off + (long long)t0 * g.stride));
-    oy[i] = (unsigned)(8LL * (a.rows[g.row0 + min(it.cb * 8 + i, g.nrows - 1)].off + (long long)t0 * g.stride));
+  for (int i = 0; i < QN; ++i) {
+    const int q = tid + T::NTH * i;
+    const int cp = 2 * (q & 7), row = (q >> 3) % R;
+    tq[i] = (q >> 3) / R;
+    on[i] = row < g.nrows && cp < nc;
+    dst[i] = (tq[i] * R + row) * RS + cp;
+    src[i] = a.spec32 + a.rows[g.row0 + min(row, g.nrows - 1)] + (long long)(t0 + tq[i]) * g.stride + it.c0 + cp;
   }
-  float2 acc[8][8];
+  float4_a8 buf[QN];
+  auto load = [&](int t) {
 #pragma unroll
-  for (int i = 0; i < 8; ++i)
-#pragma unroll
-    for (int j = 0; j < 8; ++j) acc[i][j] = make_float2(0.0f, 0.0f);
-  for (int t = t0; t < t1; ++t) {
-    float2 x[8], y[8];
-#pragma unroll
-    for (int i = 0; i < 8; ++i) {
-      const v2f vx = *(GF2)(base + (ox[i] + co));
-      const v2f vy = *(GF2)(base + (oy[i] + co));
-      x[i] = make_float2(vx.x, vx.y);
-      y[i] = make_float2(vy.x, vy.y);
-      ox[i] += st;
-      oy[i] += st;
-    }
-#pragma unroll
-    for (int i = 0; i < 8; ++i)
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        acc[i][j].x = fmaf(x[i].x, y[j].x, acc[i][j].x);
-        acc[i][j].x = fmaf(x[i].y, y[j].y, acc[i][j].x);
-        acc[i][j].y = fmaf(x[i].y, y[j].x, acc[i][j].y);
-        acc[i][j].y = fmaf(-x[i].x, y[j].y, acc[i][j].y);
-      }
-  }
-  // the partial sums of waves 1-3 through LDS, 16 entries per round
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    __syncthreads();
-    if (w > 0) {
-#pragma unroll
-      for (int k = 0; k < 16; ++k) red[w - 1][k][lane] = acc[(r * 16 + k) / 8][(r * 16 + k) % 8];
-    }
-    __syncthreads();
-    if (w == 0) {
-#pragma unroll
-      for (int k = 0; k < 16; ++k) {
-        float2 v = acc[(r * 16 + k) / 8][(r * 16 + k) % 8];
-#pragma unroll
-        for (int q = 0; q < 3; ++q) { v.x += red[q][k][lane].x; v.y += red[q][k][lane].y; }
-        acc[(r * 16 + k) / 8][(r * 16 + k) % 8] = v;
-      }
-    }
-  }
-  if (w != 0 || c >= g.C) return;
-  const int n = g.nrows;
-  const int* __restrict__ pairs = a.pairs + g.pair0;
-#pragma unroll
-  for (int i = 0; i < 8; ++i) {
-    const int ri = it.rb * 8 + i;
-    if (ri >= n) break;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const int cj = it.cb * 8 + j;
-      if (cj >= n) break;
-      const int p = pairs[ri * n + cj];
-      if (p >= 0) {
-        float2 v = acc[i][j];
-        if (ri == cj) v.y = 0.0f;
-        float2* d = a.acc + p + c;
-        *d = make_float2(d->x + v.x, d->y + v.y);
-      }
-      if (it.rb != it.cb) {
-        const int q = pairs[cj * n + ri];
-        if (q >= 0) {
-          float2* d = a.acc + q + c;
-          *d = make_float2(d->x + acc[i][j].x, d->y - acc[i][j].y);
+    for (int i = 0; i < QN; ++i) {
+      buf[i] = float4_a8{0.0f, 0.0f, 0.0f, 0.0f};
+      if (on[i] && t + tq[i] < t1) {
+        if (((tid + T::NTH * i) & 7) * 2 + 1 < nc) {
+          buf[i] = *reinterpret_cast<const float4_a8*>(src[i]);
+        } else {                                          // the window's last channel, alone
+          const float2 v = *src[i];
+          buf[i].x = v.x;
+          buf[i].y = v.y;
         }
       }
+      src[i] += (long long)TB * g.stride;
     }
+  };
+  auto store = [&](float2* d) {
+#pragma unroll
+    for (int i = 0; i < QN; ++i)
+      if (on[i]) {
+        d[dst[i]] = make_float2(buf[i].x, buf[i].y);
+        d[dst[i] + 1] = make_float2(buf[i].z, buf[i].w);
+      }
+  };
+
+  // accumulators, [channel of the wave][row tile][column tile][register]
+  typedef float accv __attribute__((ext_vector_type(NREG)));
+  accv acc[CPW][NT][NT];
+  float* part = a.part + g.off + it.split * g.split_stride + (long long)(it.c0 + wave * CPW) * T::RR + lane;
+#pragma unroll
+  for (int c = 0; c < CPW; ++c)
+#pragma unroll
+    for (int ti = 0; ti < NT; ++ti)
+#pragma unroll
+      for (int tj = 0; tj < NT; ++tj)
+#pragma unroll
+        for (int r = 0; r < NREG; ++r)
+          acc[c][ti][tj][r] = 0.0f;
+  accv tot[CPW][NT][NT];                                  // R = 64: stays zero (an empty range's sums)
+#pragma unroll
+  for (int c = 0; c < CPW; ++c)
+#pragma unroll
+    for (int ti = 0; ti < NT; ++ti)
+#pragma unroll
+      for (int tj = 0; tj < NT; ++tj) tot[c][ti][tj] = acc[c][ti][tj];
+  // the sums of a run of FFTs into the total (R = 64: into the stored accumulators, as two sets
+  // of its 64 registers per channel do not fit)
+  bool fresh = a.first;
+  auto put = [&](auto& v) {
+#pragma unroll
+    for (int c = 0; c < CPW; ++c) {
+      if (wave * CPW + c >= nc) continue;
+#pragma unroll
+      for (int ti = 0; ti < NT; ++ti)
+#pragma unroll
+        for (int tj = 0; tj < NT; ++tj)
+#pragma unroll
+          for (int r = 0; r < NREG; ++r) {
+            float* p = part + c * T::RR + (ti * NT + tj) * 1024 + r * 64;
+            *p = fresh ? v[c][ti][tj][r] : *p + v[c][ti][tj][r];
+          }
+    }
+    fresh = false;
+  };
+  auto flush = [&]() {
+    if constexpr (R == 64) put(acc);
+#pragma unroll
+    for (int c = 0; c < CPW; ++c)
+#pragma unroll
+      for (int ti = 0; ti < NT; ++ti)
+#pragma unroll
+        for (int tj = 0; tj < NT; ++tj)
+#pragma unroll
+          for (int r = 0; r < NREG; ++r) {
+            if constexpr (R != 64) tot[c][ti][tj][r] += acc[c][ti][tj][r];
+            acc[c][ti][tj][r] = 0.0f;
+          }
+  };
+
+  // lane: row l % 32 (l % 16), k = l / 32: (re, im) of one FFT, or l / 16: (re, im) of two
+  const int row = R == 16 ? lane & 15 : lane & 31;
+  const bool im = R == 16 ? (lane >> 4) & 1 : lane >> 5;
+  const int tk = R == 16 ? lane >> 5 : 0;
+  const float sgn = im ? 1.0f : -1.0f;
+  auto step = [&](const float2* s) {
+#pragma unroll
+    for (int t = 0; t < TB; t += R == 16 ? 2 : 1) {
+#pragma unroll
+      for (int c = 0; c < CPW; ++c) {
+        float av[NT], bv[NT];
+#pragma unroll
+        for (int ti = 0; ti < NT; ++ti) {
+          const float2 x = s[((t + tk) * R + row + 32 * ti) * RS + wave * CPW + c];
+          av[ti] = im ? x.y : x.x;
+          bv[ti] = fmaf(sgn, x.y, x.x);                   // re - im, re + im
+        }
+#pragma unroll
+        for (int ti = 0; ti < NT; ++ti)
+#pragma unroll
+          for (int tj = 0; tj < NT; ++tj) {
+            if constexpr (R == 16)
+              acc[c][ti][tj] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[ti], bv[tj], acc[c][ti][tj], 0, 0, 0);
+            else
+              acc[c][ti][tj] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[ti], bv[tj], acc[c][ti][tj], 0, 0, 0);
+          }
+      }
+    }
+  };
+
+  load(t0);
+  __syncthreads();
+  store(lds[0]);
+  __syncthreads();
+  int cur = 0, run = 0;
+  for (int t = t0; t < t1; t += TB, cur ^= 1) {
+    load(t + TB);                                         // past the end: zeros, not used
+    step(lds[cur]);
+    if (++run == T::RUN || t + TB >= t1) { flush(); run = 0; }
+    if (t + TB < t1) store(lds[cur ^ 1]);
+    __syncthreads();
   }
+  if (R == 64 && t0 < t1) return;                         // stored by the last flush
+  put(tot);
 }
 
 template <typename V8>
@@ -230,18 +304,19 @@ __global__ void __launch_bounds__((XTile<NTILE, CT_>::NTH)) k_xmac_mfma(XMfmaArg
     (&lds_raw[0][0])[i] = make_uint4(0u, 0u, 0u, 0u);
 
   floatx16 accr[CPW][NPAIR], acci[CPW][NPAIR];
+  float* acc0 = a.acc + g.acc_off + blockIdx.z * g.split_stride;
 #pragma unroll
   for (int cw = 0; cw < CPW; ++cw) {
     const int c = c0 + wave * CPW + cw;
-    const float* accp = a.acc + g.acc_off + (long long)c * NPAIR * 2 * 1024;
+    const float* accp = acc0 + (long long)c * NPAIR * 2 * 1024;
 #pragma unroll
     for (int p = 0; p < NPAIR; ++p) {
       const float* pr = accp + (p * 2 + 0) * 1024 + lane;    // immediate offsets r * 256 bytes
       const float* pi = accp + (p * 2 + 1) * 1024 + lane;
 #pragma unroll
       for (int r = 0; r < 16; ++r) {
-        accr[cw][p][r] = pr[r * 64];
-        acci[cw][p][r] = pi[r * 64];
+        accr[cw][p][r] = a.first ? 0.0f : pr[r * 64];
+        acci[cw][p][r] = a.first ? 0.0f : pi[r * 64];
       }
     }
   }
@@ -295,27 +370,31 @@ __global__ void __launch_bounds__((XTile<NTILE, CT_>::NTH)) k_xmac_mfma(XMfmaArg
       }
   };
 
-  const int nk = a.nffts_pad / 8;
+  // this workgroup's range of k-steps
+  const int nka = a.nffts_pad / 8;
+  const int k0 = (int)((long long)blockIdx.z * nka / g.nsplit), k1 = (int)((long long)(blockIdx.z + 1) * nka / g.nsplit);
   // one k-step of global loads in flight over a double-buffered LDS stage (two k-steps ahead
   // in registers measured slower)
   uint4 buf[QMAX];
   __syncthreads();
-  gload(0, buf);
-  lstore(lds0, buf);
+  if (k0 < k1) {                                  // uniform: a short chunk may leave a split empty
+    gload(k0, buf);
+    lstore(lds0, buf);
+  }
   __syncthreads();
-  for (int k = 0; k < nk; ++k) {
-    uint32_t* cur = (k & 1) ? lds1 : lds0;
-    uint32_t* nxt = (k & 1) ? lds0 : lds1;
-    gload(min(k + 1, nk - 1), buf);               // past the end: re-read, unused
+  for (int k = k0; k < k1; ++k) {
+    uint32_t* cur = ((k - k0) & 1) ? lds1 : lds0;
+    uint32_t* nxt = ((k - k0) & 1) ? lds0 : lds1;
+    gload(min(k + 1, k1 - 1), buf);               // past the end: re-read, unused
     mfma_step(cur);
-    if (k + 1 < nk) lstore(nxt, buf);
+    if (k + 1 < k1) lstore(nxt, buf);
     __syncthreads();
   }
 
 #pragma unroll
   for (int cw = 0; cw < CPW; ++cw) {
     const int c = c0 + wave * CPW + cw;
-    float* accp = a.acc + g.acc_off + (long long)c * NPAIR * 2 * 1024;
+    float* accp = acc0 + (long long)c * NPAIR * 2 * 1024;
 #pragma unroll
     for (int p = 0; p < NPAIR; ++p) {
       float* pr = accp + (p * 2 + 0) * 1024 + lane;
@@ -335,6 +414,114 @@ __device__ __forceinline__ int mfma_idx(int i, int j) {
   const int r = (i >> 3) * 4 + (i & 3);
   const int l = ((i >> 2) & 1) * 32 + j;
   return r * 64 + l;
+}
+// The same for a 16x16 accumulator: register r of lane l holds (4 (l / 16) + r, l % 16).
+__device__ __forceinline__ int mfma_idx16(int i, int j) { return (i & 3) * 64 + (i >> 2) * 16 + j; }
+
+// The raw accumulator tiles to the products: a workgroup reads a block of tiles of a few
+// channels of one group into LDS, whole lines at a time, summing the splits in order, and then
+// writes one value per thread with the channel fastest, so each product gets 64- or 128-byte
+// runs (read in place, the 4-byte values of one product are 1 to 16 KB apart).  A product whose
+// channels go to the results as they are is written there, the others to their accumulators.
+template <int NPL, int CH>
+__device__ __forceinline__ void xr_gather(float* s, const float* p0, const float* p1, long long chf, int nch, int len,
+                                          int cs, int nsplit, long long stride) {
+  typedef float v4 __attribute__((ext_vector_type(4)));
+  const int q4 = len / 4;                                  // len: floats per channel and plane
+#pragma unroll 2
+  for (int e = threadIdx.x; e < CH * NPL * q4; e += 256) {
+    const int ch = e / (NPL * q4), rem = e % (NPL * q4), pl = rem / q4, k = rem % q4;
+    if (ch >= nch) break;                                  // channels ascend with e
+    const v4* p = reinterpret_cast<const v4*>((NPL == 2 && pl ? p1 : p0) + ch * chf) + k;
+    v4 v = *p;
+    const long long st = stride / 4;
+    int q = 1;
+    for (; q + 4 <= nsplit; q += 4) {                      // four splits in flight
+      const v4 a = p[q * st], b = p[(q + 1) * st], c = p[(q + 2) * st], d = p[(q + 3) * st];
+      v += a; v += b; v += c; v += d;
+    }
+    for (; q < nsplit; ++q) v += p[q * st];
+    *reinterpret_cast<v4*>(s + ch * cs + pl * len + 4 * k) = v;
+  }
+}
+
+__device__ __forceinline__ void xr_put(const XReduceArgs& a, long long p, int c, float2 v) {
+  if (p >= 0) a.acc[p + c] = v;
+  else if (p < -1) a.res[-2 - p + c] = v;
+}
+
+// 16-bit X-engine: 16 channels, one pair of row tiles, eight rows (256 floats of each tile).
+constexpr int XRH_CH = 16, XRH_CS = 512 + 4;
+__global__ void __launch_bounds__(256) k_xreduce_h(XReduceArgs a) {
+  __shared__ float s[XRH_CH * XRH_CS];
+  const XRGroup g = a.groups[blockIdx.y];
+  const int c0 = blockIdx.x * XRH_CH, ntp = g.ntile * (g.ntile + 1) / 2;
+  int ti = 0, tj = blockIdx.z >> 2;
+  const int i0 = 8 * (blockIdx.z & 3), tp = tj;
+  while (tj > ti) { ++ti; tj -= ti; }
+  if (c0 >= g.C || tp >= ntp || ti * 32 + i0 >= g.n) return;
+  const int nch = min(XRH_CH, g.C - c0);
+  const long long chf = (long long)ntp * 2048;
+  const float* p = a.part + g.off + c0 * chf + (long long)tp * 2048 + i0 * 32;
+  xr_gather<2, XRH_CH>(s, p, p + 1024, chf, nch, 256, XRH_CS, g.nsplit, g.split_stride);
+  __syncthreads();
+  const int ch = threadIdx.x % XRH_CH;
+  if (ch >= nch) return;
+  const long long* pairs = a.pairs + g.pair0;
+  const float* sc = s + ch * XRH_CS;
+#pragma unroll 4
+  for (int e = threadIdx.x / XRH_CH; e < 256; e += 256 / XRH_CH) {
+    const int i = e >> 5, j = e & 31, ri = ti * 32 + i0 + i, rj = tj * 32 + j;
+    if (ri >= g.n || rj >= g.n) continue;
+    const long long p = pairs[ri * g.n + rj], q = ti == tj ? -1 : pairs[rj * g.n + ri];
+    if (p == -1 && q == -1) continue;
+    const float inv = 1.0f / (a.xscale[g.scale_off + ri] * a.xscale[g.scale_off + rj]);
+    const int k = mfma_idx(i, j);
+    float2 v = make_float2(sc[k] * inv, sc[256 + k] * inv);
+    if (ri == rj) v.y = 0.0f;                              // x conj(x) is real
+    xr_put(a, p, c0 + ch, v);
+    xr_put(a, q, c0 + ch, make_float2(v.x, -v.y));
+  }
+}
+
+// FP32 X-engine: 8 channels, one pair of row tiles: S(ti, tj) and S(tj, ti).
+constexpr int XRS_CH = 8, XRS_CS = 2048 + 8;
+__global__ void __launch_bounds__(256) k_xreduce_s(XReduceArgs a) {
+  __shared__ float s[XRS_CH * XRS_CS];
+  const XRGroup g = a.groups[blockIdx.y];
+  const int c0 = blockIdx.x * XRS_CH;
+  int ti = 0, tj = blockIdx.z;
+  while (tj > ti) { ++ti; tj -= ti; }
+  if (c0 >= g.C || ti >= g.ntile) return;
+  const bool s16 = g.kind == XR_S16;
+  const int tile = s16 ? 256 : 1024;
+  const int nch = min(XRS_CH, g.C - c0);
+  const long long chf = (long long)g.ntile * g.ntile * tile;
+  const float* p = a.part + g.off + c0 * chf;
+  if (ti == tj)
+    xr_gather<1, XRS_CH>(s, p + (long long)(ti * g.ntile + tj) * tile, nullptr, chf, nch, tile, XRS_CS, g.nsplit, g.split_stride);
+  else
+    xr_gather<2, XRS_CH>(s, p + (long long)(ti * g.ntile + tj) * tile, p + (long long)(tj * g.ntile + ti) * tile, chf, nch,
+                         tile, XRS_CS, g.nsplit, g.split_stride);
+  __syncthreads();
+  const int w = s16 ? 16 : 32, wl = s16 ? 4 : 5;
+  const int ch = threadIdx.x % XRS_CH;
+  if (ch >= nch) return;
+  const long long* pairs = a.pairs + g.pair0;
+  const float* sc = s + ch * XRS_CS;
+  const float* st = sc + (ti == tj ? 0 : tile);
+#pragma unroll 4
+  for (int e = threadIdx.x / XRS_CH; e < w * w; e += 256 / XRS_CH) {
+    const int i = e >> wl, j = e & (w - 1), ri = ti * 32 + i, rj = tj * 32 + j;
+    if (ri >= g.n || rj >= g.n) continue;
+    const long long p = pairs[ri * g.n + rj], q = ti == tj ? -1 : pairs[rj * g.n + ri];
+    if (p == -1 && q == -1) continue;
+    const float x = sc[s16 ? mfma_idx16(i, j) : mfma_idx(i, j)];
+    const float y = st[s16 ? mfma_idx16(j, i) : mfma_idx(j, i)];
+    const float2 v = make_float2(0.5f * (x + y), 0.5f * (x - y));   // i = j: imaginary part 0
+    xr_put(a, p, c0 + ch, v);
+    xr_put(a, q, c0 + ch, make_float2(v.x, -v.y));
+  }
 }
 
 // ---- accumulation into the slot results (core.cpp:1819-1853, 1258-1376) ----------------
@@ -362,8 +549,8 @@ __device__ __forceinline__ float2 uv_rotate(float2 v, double dd, const UvFreq& q
   return make_float2(r.x * c2 - r.y * s2, r.x * s2 + r.y * c2);
 }
 
-__global__ void k_fin_plain(const FinPlain* e, const float2* acc, float2* res, UvArgs uv) {
-  const FinPlain f = e[blockIdx.y];
+__global__ void k_fin(const FinProd* e, const float2* acc, float2* res, UvArgs uv) {
+  const FinProd f = e[blockIdx.y];
   const int co = blockIdx.x * blockDim.x + threadIdx.x;
   if (co >= f.nout) return;
   if (uv.P > 1 && f.bl >= 0) {                    // rotated into every phase centre's block
@@ -395,55 +582,6 @@ __global__ void k_fin_plain(const FinPlain* e, const float2* acc, float2* res, U
   res[f.dst + co] = o;
 }
 
-
-__global__ void k_fin_mfma(const FinMfma* e, const DevXGroup* groups, const float* acc,
-                           const float* xscale, float2* res, UvArgs uv) {
-  const FinMfma f = e[blockIdx.y];
-  const int co = blockIdx.x * blockDim.x + threadIdx.x;
-  if (co >= f.nout) return;
-  const DevXGroup g = groups[f.group];
-  const int npair = g.ntile * (g.ntile + 1) / 2;
-  int r1 = f.row1, r2 = f.row2;
-  float sign = 1.0f;
-  int ti = r1 >> 5, tj = r2 >> 5;
-  if (ti < tj) { int tmp = r1; r1 = r2; r2 = tmp; ti = r1 >> 5; tj = r2 >> 5; sign = -1.0f; }
-  const int pair = ti * (ti + 1) / 2 + tj;
-  const int idx = mfma_idx(r1 & 31, r2 & 31);
-  if (uv.P > 1 && f.bl >= 0) {                    // rotated into every phase centre's block
-    const UvFreq q = uv.fq[f.fq];
-    const float inv = 1.0f / (xscale[g.scale_off + f.row1] * xscale[g.scale_off + f.row2]);
-    for (int p = 0; p < uv.P; ++p) {
-      const double dd = uv.dd[f.bl * uv.P + p];
-      const bool turn = fabs(dd) > 1.0e-20;
-      float2 s = make_float2(0.f, 0.f);
-      for (int k = 0; k < f.avg; ++k) {
-        const int ch = co * f.avg + k;
-        const float* base = acc + g.acc_off + ((long long)(f.chan0 + ch) * npair + pair) * 2 * 1024;
-        float2 v = make_float2(base[idx] * inv, sign * base[1024 + idx] * inv);
-        if (turn) v = uv_rotate(v, dd, q, ch);
-        s.x += v.x; s.y += v.y;
-      }
-      if (f.avg > 1) { s.x /= (float)f.avg; s.y /= (float)f.avg; }
-      float2* o = res + f.dst + (long long)p * f.pcstride + co;
-      o->x += s.x; o->y += s.y;
-    }
-    return;
-  }
-  float2 s = make_float2(0.f, 0.f);
-  for (int k = 0; k < f.avg; ++k) {
-    const int c = f.chan0 + co * f.avg + k;
-    const float* base = acc + g.acc_off + ((long long)c * npair + pair) * 2 * 1024;
-    const float sc = xscale[g.scale_off + f.row1] * xscale[g.scale_off + f.row2];
-    const float inv = 1.0f / sc;
-    s.x += base[idx] * inv;
-    s.y += sign * base[1024 + idx] * inv;
-  }
-  if (f.avg > 1) { s.x /= (float)f.avg; s.y /= (float)f.avg; }
-  if (f.isauto) s.y = 0.0f;
-  float2 o = res[f.dst + co];
-  o.x += s.x; o.y += s.y;
-  res[f.dst + co] = o;
-}
 
 // Baseline weights (core.cpp:1005-1052, 1066-1112) and autocorrelation weights
 // (core.cpp:1306-1370): sequential FP32 sums over the FFTs of the subint.
@@ -488,9 +626,20 @@ __global__ void k_fill(float* p, long long n, float v) {
 }
 
 // ---- host-side launchers -------------------------------------------------------------
-int fxg_launch_xplain_blk(const XPBlkArgs& a, int nitems, hipStream_t st) {
-  if (nitems == 0) return 0;
-  hipLaunchKernelGGL(k_xmac_f32_blk, dim3(nitems), dim3(256), 0, st, a);
+int fxg_launch_xplain_mat(const XPMatArgs& a, int R, int nitems, hipStream_t st) {
+  const dim3 grid(nitems);
+  if (R == 16) hipLaunchKernelGGL(k_xmac_f32_mat<16>, grid, dim3(XPTile<16>::NTH), 0, st, a);
+  else if (R == 32) hipLaunchKernelGGL(k_xmac_f32_mat<32>, grid, dim3(XPTile<32>::NTH), 0, st, a);
+  else hipLaunchKernelGGL(k_xmac_f32_mat<64>, grid, dim3(XPTile<64>::NTH), 0, st, a);
+  return hipGetLastError() == hipSuccess ? 0 : -1;
+}
+
+int fxg_launch_xreduce(const XReduceArgs& a, int mfma, int ngroups, int maxC, int maxtp, hipStream_t st) {
+  if (ngroups == 0) return 0;
+  if (mfma)
+    hipLaunchKernelGGL(k_xreduce_h, dim3((maxC + XRH_CH - 1) / XRH_CH, ngroups, 4 * maxtp), dim3(256), 0, st, a);
+  else
+    hipLaunchKernelGGL(k_xreduce_s, dim3((maxC + XRS_CH - 1) / XRS_CH, ngroups, maxtp), dim3(256), 0, st, a);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
@@ -501,46 +650,41 @@ int fxg_launch_xplain(const XPlainArgs& a, int nprod, int maxchan, hipStream_t s
 }
 
 template <typename V8, int NTILE, int CT>
-static void launch_x(const XMfmaArgs& b, int C, int ngroups, hipStream_t st) {
-  hipLaunchKernelGGL((k_xmac_mfma<V8, NTILE, CT>), dim3(C / CT, ngroups), dim3(XTile<NTILE, CT>::NTH), 0, st, b);
+static void launch_x(const XMfmaArgs& b, int C, int ngroups, int nsplit, hipStream_t st) {
+  hipLaunchKernelGGL((k_xmac_mfma<V8, NTILE, CT>), dim3(C / CT, ngroups, nsplit), dim3(XTile<NTILE, CT>::NTH), 0, st, b);
 }
 
-// groups [group0, group0 + ngroup_launch) share the tile count, channel count and tile width
-int fxg_launch_xmfma(const XMfmaArgs& a, int ngroup_launch, int group0, int ntile, int C, int twlog, hipStream_t st) {
+// groups [group0, group0 + ngroup_launch) share the tile count, channel count, tile width and
+// splits of g
+int fxg_launch_xmfma(const XMfmaArgs& a, int ngroup_launch, int group0, const DevXGroup& g, hipStream_t st) {
   XMfmaArgs b = a;
+  const int ntile = g.ntile, C = g.C, twlog = g.twlog, ns = g.nsplit;
   b.groups = a.groups + group0;
   const int ct = 1 << twlog;
   if (C % ct || (ct != 8 && ct != 16) || (ntile != 1 && ntile != 2) || (ntile == 2 && ct != 8)) return -2;
   const int form = (a.mode == 1 ? 0 : 4) + (ntile == 1 ? 0 : 2) + (ct == 8 ? 0 : 1);
   switch (form) {
-    case 0: launch_x<half8_t, 1, 8>(b, C, ngroup_launch, st); break;
-    case 1: launch_x<half8_t, 1, 16>(b, C, ngroup_launch, st); break;
-    case 2: launch_x<half8_t, 2, 8>(b, C, ngroup_launch, st); break;
-    case 4: launch_x<bf16x8_t, 1, 8>(b, C, ngroup_launch, st); break;
-    case 5: launch_x<bf16x8_t, 1, 16>(b, C, ngroup_launch, st); break;
-    case 6: launch_x<bf16x8_t, 2, 8>(b, C, ngroup_launch, st); break;
+    case 0: launch_x<half8_t, 1, 8>(b, C, ngroup_launch, ns, st); break;
+    case 1: launch_x<half8_t, 1, 16>(b, C, ngroup_launch, ns, st); break;
+    case 2: launch_x<half8_t, 2, 8>(b, C, ngroup_launch, ns, st); break;
+    case 4: launch_x<bf16x8_t, 1, 8>(b, C, ngroup_launch, ns, st); break;
+    case 5: launch_x<bf16x8_t, 1, 16>(b, C, ngroup_launch, ns, st); break;
+    case 6: launch_x<bf16x8_t, 2, 8>(b, C, ngroup_launch, ns, st); break;
     default: return -2;
   }
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-int fxg_launch_fin_plain(const FinPlain* e, int n, int maxout, const float2* acc, float2* res, const UvArgs& uv,
+int fxg_launch_fin(const FinProd* e, int n, int maxout, const float2* acc, float2* res, const UvArgs& uv,
                          hipStream_t st) {
   if (n == 0) return 0;
-  hipLaunchKernelGGL(k_fin_plain, dim3((maxout + 255) / 256, n), dim3(256), 0, st, e, acc, res, uv);
+  hipLaunchKernelGGL(k_fin, dim3((maxout + 255) / 256, n), dim3(256), 0, st, e, acc, res, uv);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 int fxg_launch_add_at(const int* idx, const float* val, int n, float* resf, hipStream_t st) {
   if (n == 0) return 0;
   hipLaunchKernelGGL(k_add_at, dim3((n + 255) / 256), dim3(256), 0, st, idx, val, n, resf);
-  return hipGetLastError() == hipSuccess ? 0 : -1;
-}
-
-int fxg_launch_fin_mfma(const FinMfma* e, int n, int maxout, const DevXGroup* g, const float* acc,
-                        const float* xscale, float2* res, const UvArgs& uv, hipStream_t st) {
-  if (n == 0) return 0;
-  hipLaunchKernelGGL(k_fin_mfma, dim3((maxout + 255) / 256, n), dim3(256), 0, st, e, g, acc, xscale, res, uv);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
