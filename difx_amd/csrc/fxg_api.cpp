@@ -1032,7 +1032,7 @@ int x_splits(const fxg_ctx* ctx, long long units, long long wanted) {
 // The matrix plain X-engine's tables.  A row is a spectra band or zoom window with its channel
 // count, (datastream, band, channel offset, channels); products join rows into groups.  Each
 // group of at most 64 rows gets a pair table (the accumulator of the product of rows (i, j), or
-// -1) and work items of XP_CT channels.  Products of groups above 64 rows or whose rows'
+// -1) and work items of xp_ct channels.  Products of groups above 64 rows or whose rows'
 // datastreams differ in FFT stride, and a second product of the same row pair, stay with the
 // per-product kernel.  Returns the floats of raw accumulator tiles.
 long long build_xplain(fxg_ctx* ctx) {
@@ -1113,15 +1113,15 @@ long long build_xplain(fxg_ctx* ctx) {
   // 30.5 ms
   long long off = 0;
   for (int R : {16, 32, 64}) {
-    auto cls = [&](const XPGroup& G) { return G.nrows <= 16 ? 16 : G.nrows <= 32 ? 32 : 64; };
+    const int ct = xp_ct(R);
     long long units = 0;
-    for (const auto& G : ctx->xp_groups) if (cls(G) == R) units += (G.C + XP_CT - 1) / XP_CT;
+    for (const auto& G : ctx->xp_groups) if (xp_class(G.nrows) == R) units += (G.C + ct - 1) / ct;
     if (!units) continue;
     const int ns = x_splits(ctx, units, 4LL * ctx->ncu);
     const int item0 = (int)ctx->xp_items.size();
     for (size_t gi = 0; gi < ctx->xp_groups.size(); ++gi) {
       XPGroup& G = ctx->xp_groups[gi];
-      if (cls(G) != R) continue;
+      if (xp_class(G.nrows) != R) continue;
       G.off = off;
       G.split_stride = (long long)G.C * R * R;
       G.nsplit = ns;
@@ -1130,8 +1130,12 @@ long long build_xplain(fxg_ctx* ctx) {
       X.off = G.off;
       X.split_stride = G.split_stride;
       X.nsplit = ns;
+      // workgroups go to the eight XCDs in turn: the two 8-channel items of a 128-byte line are
+      // placed eight apart, so that they share an XCD's L2
       for (int q = 0; q < ns; ++q)
-        for (int c0 = 0; c0 < G.C; c0 += XP_CT) ctx->xp_items.push_back(XPItem{(int)gi, c0, q});
+        for (int c = 0; c < G.C; c += 8 * 16)
+          for (int h = 0; h < 16; h += ct)
+            for (int c0 = c + h; c0 < std::min(G.C, c + 8 * 16); c0 += 16) ctx->xp_items.push_back(XPItem{(int)gi, c0, q});
     }
     ctx->xp_classes.push_back({R, item0, (int)ctx->xp_items.size() - item0});
   }
@@ -1233,13 +1237,22 @@ int build_engines(fxg_ctx* ctx, int chunk_req) {
   ctx->chunkcap = (int)cap;
   if (int rc_ = dev_malloc(ctx, (void**)&ctx->d_params, sizeof(FftDelay) * (size_t)nds * cap)) return rc_;
   if (mfma) {
+    // Split each launch's FFT loop (groups of one shape run together) so that it has two
+    // workgroups per CU: 32 stations x 256 channels (64 channel tiles) 2000 -> 1280 us per subint;
+    // four or eight per CU cost more in accumulator traffic than they gain (1316, 1395 us).
+    for (size_t g0 = 0, g1; g0 < ctx->groups.size(); g0 = g1) {
+      const DevXGroup& G = ctx->groups[g0];
+      for (g1 = g0; g1 < ctx->groups.size() && ctx->groups[g1].ntile == G.ntile && ctx->groups[g1].C == G.C; ++g1) {}
+      const long long units = (long long)(g1 - g0) * (G.C >> G.twlog);
+      const int ns = x_splits(ctx, units, 2LL * ctx->ncu);
+      for (size_t g = g0; g < g1; ++g) ctx->groups[g].nsplit = ns;
+    }
     long long off = 0, aoff = 0, soff = 0;
     for (auto& g : ctx->groups) {
       g.spec_off = off;
       g.rowstride = cap * g.C + 32;       // one 128-byte line of padding per row
       off += (long long)g.ntile * 32 * g.rowstride;
       g.split_stride = (long long)g.C * (g.ntile * (g.ntile + 1) / 2) * 2 * 1024;
-      g.nsplit = 1;
       g.acc_off = aoff;
       aoff += g.nsplit * g.split_stride;
       g.scale_off = soff;
@@ -1354,7 +1367,6 @@ int build_engines(fxg_ctx* ctx, int chunk_req) {
       }
     }
     ctx->xacc_len = acc;
-    if (int rc_ = dev_malloc(ctx, (void**)&ctx->d_xacc, sizeof(float2) * std::max<long long>(acc, 2))) return rc_;
     const long long plen = build_xplain(ctx);
     if (!ctx->xp_items.empty()) {
       if (int rc = dev_malloc(ctx, (void**)&ctx->d_vacc, (long long)sizeof(float) * plen)) return rc;
@@ -1446,33 +1458,29 @@ int build_engines(fxg_ctx* ctx, int chunk_req) {
       }
     }
     ctx->xacc_len = acc;
-    if (int rc = dev_malloc(ctx, (void**)&ctx->d_xacc, (long long)sizeof(float2) * std::max<long long>(acc, 2))) return rc;
   }
   // products that go to the results channel by channel (one phase centre, no averaging, no other
   // reader such as a zoom window) are written there by the reduction itself
   if (ctx->nphase <= 1) {
-    std::map<long long, std::pair<long long*, int>> slot;          // accumulator -> entry, channels
+    struct PairSlot { long long acc; long long* entry; int C, readers; };
+    std::vector<PairSlot> slot;
     for (const auto& X : ctx->xr_groups)
       for (int k = 0; k < X.n * X.n; ++k)
-        if (ctx->xr_pairs[X.pair0 + k] >= 0) slot[ctx->xr_pairs[X.pair0 + k]] = {&ctx->xr_pairs[X.pair0 + k], X.C};
-    std::map<long long, int> readers;
-    auto of = [&](long long src) {
-      auto it = slot.upper_bound(src);
-      if (it == slot.begin()) return slot.end();
+        if (ctx->xr_pairs[X.pair0 + k] >= 0) slot.push_back({ctx->xr_pairs[X.pair0 + k], &ctx->xr_pairs[X.pair0 + k], X.C, 0});
+    std::sort(slot.begin(), slot.end(), [](const PairSlot& a, const PairSlot& b) { return a.acc < b.acc; });
+    auto of = [&](long long src) -> PairSlot* {
+      auto it = std::upper_bound(slot.begin(), slot.end(), src, [](long long v, const PairSlot& s) { return v < s.acc; });
+      if (it == slot.begin()) return nullptr;
       --it;
-      return src < it->first + it->second.second ? it : slot.end();
+      return src < it->acc + it->C ? &*it : nullptr;
     };
-    for (const auto& e : ctx->finp) {
-      auto it = of(e.src);
-      if (it != slot.end()) readers[it->first]++;
-    }
+    for (const auto& e : ctx->finp)
+      if (PairSlot* s = of(e.src)) s->readers++;
     std::vector<FinProd> rest;
     for (const auto& e : ctx->finp) {
-      auto it = of(e.src);
-      if (it != slot.end() && it->first == e.src && readers[e.src] == 1 && e.avg == 1 && e.nout == it->second.second)
-        *it->second.first = -2 - (long long)e.dst;
-      else
-        rest.push_back(e);
+      PairSlot* s = of(e.src);
+      if (s && s->acc == e.src && s->readers == 1 && e.avg == 1 && e.nout == s->C) *s->entry = -2 - (long long)e.dst;
+      else rest.push_back(e);
     }
     ctx->finp.swap(rest);
   }
@@ -1480,6 +1488,8 @@ int build_engines(fxg_ctx* ctx, int chunk_req) {
     ctx->xr_maxC = std::max(ctx->xr_maxC, X.C);
     ctx->xr_maxtp = std::max(ctx->xr_maxtp, X.ntile * (X.ntile + 1) / 2);
   }
+  if (ctx->finp.empty()) ctx->xacc_len = 0;        // nothing reads a product accumulator
+  if (int rc = dev_malloc(ctx, (void**)&ctx->d_xacc, (long long)sizeof(float2) * std::max<long long>(ctx->xacc_len, 2))) return rc;
   if (int rc = dev_upload(ctx, &ctx->d_finp, ctx->finp)) return rc;
   if (int rc = dev_upload(ctx, &ctx->d_xr_groups, ctx->xr_groups)) return rc;
   if (int rc = dev_upload(ctx, &ctx->d_xr_pairs, ctx->xr_pairs)) return rc;

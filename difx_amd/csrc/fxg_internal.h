@@ -217,9 +217,10 @@ struct XPlainArgs {
 
 // Plain FP32 X-engine on FP32 matrix instructions.  A group is a set of rows (spectra bands,
 // or zoom windows of them, with one channel count and FFT stride) that products connect; a work
-// item is XP_CT consecutive channels of one group.
-#define XP_CT 16            // channels per work item
+// item is xp_ct(R) consecutive channels of one group, R its row class.
 #define XP_MAXROWS 64       // rows per group (larger groups: per-product kernel)
+constexpr int xp_class(int nrows) { return nrows <= 16 ? 16 : nrows <= 32 ? 32 : 64; }
+constexpr int xp_ct(int R) { return R == 64 ? 8 : 16; }
 struct XPGroup {
   int nrows, C, row0;       // rows[row0 + i]: cf32 offset of (band, FFT 0, window start)
   int stride;               // cf32 entries between consecutive FFTs, the same for every row

@@ -62,26 +62,27 @@ __global__ void __launch_bounds__(256) k_xmac_f32(XPlainArgs a) {
 //   re V = (S + S^T) / 2,  im V = (S - S^T) / 2
 // (re V is symmetric and im V antisymmetric), so one FP32 matrix instruction per FFT does the
 // work of a real and an imaginary one.  Inputs, products and sums stay FP32.
-// A workgroup takes XP_CT channels of one group (one 128-byte line per row and FFT) and a range
+// A workgroup takes 16 channels (8 for R = 64) of one group, a line per row and FFT, and a range
 // of the chunk's FFTs; TB FFTs at a time are staged in LDS as [FFT][row][channel] (one pad entry
 // per row: a wave's reads, one row per lane, then hit distinct banks), double buffered, the next
 // stage's loads in flight while the current one is multiplied.  Rows past the group stay zero.
-// Runs of 256 FFTs (512 for R = 64) are summed apart and then added to the total: one chain over
-// 7800 FFTs of 10 stations was 1.3e-6 off the 64-bit result, against 1.8e-7 in quarters of a chunk.
+// Runs of 64 FFTs are summed apart and then added to the total: one chain over 7800 FFTs of 10
+// stations was 1.3e-6 off the 64-bit result, runs of 256 1.1e-7.
 // R is the row count rounded up to 16, 32 or 64 (16x16x4 tiles, else 32x32x2).
 template <int R>
 struct XPTile {
-  static constexpr int NTH = 16 * R;                      // waves of 4, 2 or 1 channels: the accumulators
-                                                          // of a channel are 8, 32 or 64 registers
+  static constexpr int CT = R == 64 ? 8 : 16;             // channels
+  static constexpr int NTH = R == 16 ? 256 : 512;
   static constexpr int NW = NTH / 64;
-  static constexpr int CPW = XP_CT / NW;                  // channels per wave
-  static constexpr int TB = 128 / R;                      // FFTs per stage
-  static constexpr int RS = XP_CT + 1;                    // LDS entries per row
+  static constexpr int CPW = CT / NW;                     // channels per wave: its sums and totals
+                                                          // are 32 (R = 16), 64 or 128 registers
+  static constexpr int TB = R == 64 ? 4 : 128 / R;        // FFTs per stage
+  static constexpr int RS = CT + 1;                       // LDS entries per row
   static constexpr int STAGE = TB * R * RS;
-  static constexpr int QN = TB * R * (XP_CT / 2) / NTH;   // 16-byte loads per thread and stage
+  static constexpr int QN = TB * R * (CT / 2) / NTH;      // 16-byte loads per thread and stage
   static constexpr int NT = R == 64 ? 2 : 1;              // row tiles
   static constexpr int RR = R * R;                        // accumulators per channel
-  static constexpr int RUN = (R == 64 ? 512 : 256) / TB;  // stages summed before they join the total
+  static constexpr int RUN = 64 / TB;                     // stages summed before they join the total
 };
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float float4_a8 __attribute__((ext_vector_type(4), aligned(8)));
@@ -101,15 +102,15 @@ __global__ void __launch_bounds__(XPTile<R>::NTH) k_xmac_f32_mat(XPMatArgs a) {
 
   for (int i = tid; i < 2 * T::STAGE; i += T::NTH) (&lds[0][0])[i] = make_float2(0.0f, 0.0f);
 
-  // load q of a stage: FFT q / (8 R), row (q / 8) % R, channels 2 (q % 8) and the next
+  // load q of a stage, channel pair fastest, then row, then FFT
   const float2* src[QN];
   bool on[QN];
   int tq[QN], dst[QN];
 #pragma unroll
   for (int i = 0; i < QN; ++i) {
     const int q = tid + T::NTH * i;
-    const int cp = 2 * (q & 7), row = (q >> 3) % R;
-    tq[i] = (q >> 3) / R;
+    const int cp = 2 * (q % (T::CT / 2)), row = q / (T::CT / 2) % R;
+    tq[i] = q / (T::CT / 2) / R;
     on[i] = row < g.nrows && cp < nc;
     dst[i] = (tq[i] * R + row) * RS + cp;
     src[i] = a.spec32 + a.rows[g.row0 + min(row, g.nrows - 1)] + (long long)(t0 + tq[i]) * g.stride + it.c0 + cp;
@@ -120,7 +121,7 @@ __global__ void __launch_bounds__(XPTile<R>::NTH) k_xmac_f32_mat(XPMatArgs a) {
     for (int i = 0; i < QN; ++i) {
       buf[i] = float4_a8{0.0f, 0.0f, 0.0f, 0.0f};
       if (on[i] && t + tq[i] < t1) {
-        if (((tid + T::NTH * i) & 7) * 2 + 1 < nc) {
+        if ((tid + T::NTH * i) % (T::CT / 2) * 2 + 1 < nc) {
           buf[i] = *reinterpret_cast<const float4_a8*>(src[i]);
         } else {                                          // the window's last channel, alone
           const float2 v = *src[i];
@@ -153,46 +154,13 @@ __global__ void __launch_bounds__(XPTile<R>::NTH) k_xmac_f32_mat(XPMatArgs a) {
 #pragma unroll
         for (int r = 0; r < NREG; ++r)
           acc[c][ti][tj][r] = 0.0f;
-  accv tot[CPW][NT][NT];                                  // R = 64: stays zero (an empty range's sums)
+  accv tot[CPW][NT][NT];
 #pragma unroll
   for (int c = 0; c < CPW; ++c)
 #pragma unroll
     for (int ti = 0; ti < NT; ++ti)
 #pragma unroll
       for (int tj = 0; tj < NT; ++tj) tot[c][ti][tj] = acc[c][ti][tj];
-  // the sums of a run of FFTs into the total (R = 64: into the stored accumulators, as two sets
-  // of its 64 registers per channel do not fit)
-  bool fresh = a.first;
-  auto put = [&](auto& v) {
-#pragma unroll
-    for (int c = 0; c < CPW; ++c) {
-      if (wave * CPW + c >= nc) continue;
-#pragma unroll
-      for (int ti = 0; ti < NT; ++ti)
-#pragma unroll
-        for (int tj = 0; tj < NT; ++tj)
-#pragma unroll
-          for (int r = 0; r < NREG; ++r) {
-            float* p = part + c * T::RR + (ti * NT + tj) * 1024 + r * 64;
-            *p = fresh ? v[c][ti][tj][r] : *p + v[c][ti][tj][r];
-          }
-    }
-    fresh = false;
-  };
-  auto flush = [&]() {
-    if constexpr (R == 64) put(acc);
-#pragma unroll
-    for (int c = 0; c < CPW; ++c)
-#pragma unroll
-      for (int ti = 0; ti < NT; ++ti)
-#pragma unroll
-        for (int tj = 0; tj < NT; ++tj)
-#pragma unroll
-          for (int r = 0; r < NREG; ++r) {
-            if constexpr (R != 64) tot[c][ti][tj][r] += acc[c][ti][tj][r];
-            acc[c][ti][tj][r] = 0.0f;
-          }
-  };
 
   // lane: row l % 32 (l % 16), k = l / 32: (re, im) of one FFT, or l / 16: (re, im) of two
   const int row = R == 16 ? lane & 15 : lane & 31;
@@ -232,12 +200,36 @@ __global__ void __launch_bounds__(XPTile<R>::NTH) k_xmac_f32_mat(XPMatArgs a) {
   for (int t = t0; t < t1; t += TB, cur ^= 1) {
     load(t + TB);                                         // past the end: zeros, not used
     step(lds[cur]);
-    if (++run == T::RUN || t + TB >= t1) { flush(); run = 0; }
+    if (++run == T::RUN || t + TB >= t1) {
+      run = 0;
+#pragma unroll
+      for (int c = 0; c < CPW; ++c)
+#pragma unroll
+        for (int ti = 0; ti < NT; ++ti)
+#pragma unroll
+          for (int tj = 0; tj < NT; ++tj)
+#pragma unroll
+            for (int r = 0; r < NREG; ++r) {
+              tot[c][ti][tj][r] += acc[c][ti][tj][r];
+              acc[c][ti][tj][r] = 0.0f;
+            }
+    }
     if (t + TB < t1) store(lds[cur ^ 1]);
     __syncthreads();
   }
-  if (R == 64 && t0 < t1) return;                         // stored by the last flush
-  put(tot);
+#pragma unroll
+  for (int c = 0; c < CPW; ++c) {
+    if (wave * CPW + c >= nc) continue;
+#pragma unroll
+    for (int ti = 0; ti < NT; ++ti)
+#pragma unroll
+      for (int tj = 0; tj < NT; ++tj)
+#pragma unroll
+        for (int r = 0; r < NREG; ++r) {
+          float* p = part + c * T::RR + (ti * NT + tj) * 1024 + r * 64;
+          *p = a.first ? tot[c][ti][tj][r] : *p + tot[c][ti][tj][r];
+        }
+  }
 }
 
 template <typename V8>
