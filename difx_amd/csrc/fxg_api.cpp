@@ -105,6 +105,7 @@ struct fxg_ctx {
     bool big = false;            // L > FXG_MAX_L: four-step F-engine
     long long twL_off = 0;       // big: exp(-2 pi i j / L), j < L
     int wgx = 1;                 // big: workgroups per datastream (scratch rows)
+    bool mat = false;            // the matrix F-engine takes it (see build_tables)
   };
   float2* d_bigscratch = nullptr;
   int bigL = 0;
@@ -115,7 +116,9 @@ struct fxg_ctx {
     int mode = FXG_F_PER_LENGTH;
     int ntb = 0;                 // workgroup size; 0 = 256 below L = 4096, 512 from there
     int grid_mult = 1;           // persistent: workgroups per CU
+    bool mat = false;            // the matrix F-engine where it applies
   };
+  uint32_t* d_fmat = nullptr;    // its constant tables
   FChoice fsel;
   int cfg_fmode = 0, cfg_fthreads = 0, cfg_autotune = 0;
   std::vector<std::pair<std::string, double>> tune_log;   // candidate, ms per subint (< 0: failed)
@@ -964,6 +967,23 @@ int build_tables(fxg_ctx* ctx) {
     const DevDs& x = ctx->h_ds[d];
     const int need = (std::max(x.S + x.NS, x.S + x.NFS) + 7) / 8 * 8;
     ctx->fclasses[k].phcap = std::max(ctx->fclasses[k].phcap, need);
+  }
+  // The matrix F-engine takes 2048-point FFTs of 2-bit samples whose rotator phase is linear in
+  // the sample (orders 0 and 1): its first stage needs samples of few levels and a separable
+  // rotator.
+  bool anymat = false;
+  for (auto& c : ctx->fclasses) {
+    c.mat = c.L == 2048 && !c.cplx && ctx->rotorder != 2;
+    for (int d : c.dsl) c.mat = c.mat && ctx->h_ds[d].nbits == 2;
+    anymat = anymat || c.mat;
+  }
+  if (anymat) {
+    static const std::vector<uint32_t> t = [] {   // the same for every context
+      std::vector<uint32_t> v(FMAT_TABLE_WORDS);
+      fxg_fmat_tables(v.data());
+      return v;
+    }();
+    if ((rc = dev_upload(ctx, &ctx->d_fmat, t))) return rc;
   }
   // FFT twiddles of the Stockham passes after the first, per pass (R, Ns): entries
   // exp(-2 pi i k r / (Ns R)) for r = 1..R-1, k = 0..Ns-1, k fastest; computed in FP64.
@@ -1839,6 +1859,13 @@ int launch_fengines(fxg_ctx* ctx, FengineArgs& fa, hipStream_t st) {
   for (const auto& fc : ctx->fclasses) {
     if (fc.big) continue;
     const int ncl = (int)fc.dsl.size();
+    if (ctx->fsel.mat && fc.mat) {
+      fa.dslist = ctx->d_dslist + fc.dsl_off;
+      int nfr = 1;
+      for (int d : fc.dsl) nfr = std::max(nfr, ctx->h_ds[d].nrecfreqs);
+      if (fxg_launch_fmat(fa, ncl, ctx->ncu, nfr, ctx->d_fmat, st)) return fail(ctx, FXG_E_HIP, "F-engine launch");
+      continue;
+    }
     // enough workgroups to fill the CUs several times over
     const long long wgs_per_ds = std::max(1LL, (long long)(8 * ctx->ncu + ncl - 1) / ncl);
     fa.units_per_wg = (int)std::max(1LL, std::min<long long>(8, nunits / wgs_per_ds));
@@ -2117,6 +2144,12 @@ int autotune(fxg_ctx* ctx) {
     c.grid_mult = mult;
     cand.emplace_back(name, c);
   };
+  for (const auto& fc : ctx->fclasses)
+    if (fc.mat && ctx->cfg_fmode == FXG_F_AUTO && !ctx->cfg_fthreads) {
+      add("matrix where it applies, else per-length, 256/512 threads by length", FXG_F_PER_LENGTH, 0, 1);
+      cand.back().second.mat = true;
+      break;
+    }
   add("per-length, 256/512 threads by length", FXG_F_PER_LENGTH, 0, 1);
   add("per-length, 256 threads", FXG_F_PER_LENGTH, 256, 1);
   add("per-length, 512 threads", FXG_F_PER_LENGTH, 512, 1);
@@ -2221,7 +2254,7 @@ int autotune(fxg_ctx* ctx) {
 void free_ctx(fxg_ctx* ctx) {
   auto f = [](void* p) { if (p) (void)hipFree(p); };
   f(ctx->d_ds); f(ctx->d_run); f(ctx->d_model); f(ctx->d_chanfreq); f(ctx->d_fvalid); f(ctx->d_fzone);
-  f(ctx->d_twiddle); f(ctx->d_dslist); f(ctx->d_params); f(ctx->d_items[0]); f(ctx->d_items[1]);
+  f(ctx->d_twiddle); f(ctx->d_fmat); f(ctx->d_dslist); f(ctx->d_params); f(ctx->d_items[0]); f(ctx->d_items[1]);
   f(ctx->d_iclass[0]); f(ctx->d_iclass[1]);
   f(ctx->d_counter); f(ctx->d_bigscratch); f(ctx->d_weights); f(ctx->d_flags); f(ctx->d_spec32); f(ctx->d_spec16);
   f(ctx->d_xp_groups); f(ctx->d_xp_rows); f(ctx->d_xp_items); f(ctx->d_xr_groups); f(ctx->d_xr_pairs);
@@ -2539,6 +2572,7 @@ int create_impl(const fxg_config* cfg, fxg_ctx** out, bool dry) {
   ctx->cfg_autotune = cfg->autotune;
   ctx->fsel.mode = cfg->fengine_mode == FXG_F_PERSISTENT ? FXG_F_PERSISTENT : FXG_F_PER_LENGTH;
   ctx->fsel.ntb = cfg->fengine_threads;
+  ctx->fsel.mat = cfg->fengine_mode == FXG_F_AUTO && !cfg->fengine_threads;
   if (!dry) (void)hipDeviceGetAttribute(&ctx->ncu, hipDeviceAttributeMultiprocessorCount, ctx->device);
   int rc = validate_and_derive(ctx);
   if (rc == FXG_OK) {
@@ -3264,7 +3298,7 @@ int fxg_delay_interpolator(fxg_ctx* ctx, int32_t ds, int32_t sec, int32_t ns, do
 int fxg_autotune_report(const fxg_ctx* ctx, char* buf, int32_t len) {
   if (!ctx || !buf || len < 1) return FXG_E_INVALID;
   std::string r = "F-engine: ";
-  r += ctx->fsel.mode == FXG_F_PERSISTENT ? "persistent" : "per-length";
+  r += ctx->fsel.mode == FXG_F_PERSISTENT ? "persistent" : ctx->fsel.mat ? "matrix where it applies, else per-length" : "per-length";
   r += ", threads " + (ctx->fsel.ntb ? std::to_string(ctx->fsel.ntb) : std::string("by length"));
   if (ctx->fsel.mode == FXG_F_PERSISTENT) r += ", " + std::to_string(ctx->fsel.grid_mult) + " workgroup(s)/CU";
   for (const auto& e : ctx->tune_log) {

@@ -322,6 +322,13 @@ size_t fxg_fengine_lds(int L, int ntb, int phcap, int order);
 int fxg_launch_fbig(const FengineArgs& a, int L, int iscomplex, int nds, int wgx, float2* scratch,
                     const float2* twL, hipStream_t st);
 size_t fxg_fbig_lds(int ntb, int phcap);
+// Matrix F-engine (fxg_fmat.hip): words of its constant tables and their three parts.
+constexpr int FMAT_W_WORDS = 2 * 4 * 2 * 64 * 4;
+constexpr int FMAT_T_WORDS = 2 * 16 * 64 * 2;
+constexpr int FMAT_M_WORDS = 2 * 2 * 4 * 64 * 4;
+constexpr int FMAT_TABLE_WORDS = FMAT_W_WORDS + FMAT_T_WORDS + FMAT_M_WORDS;
+void fxg_fmat_tables(uint32_t* out);
+int fxg_launch_fmat(const FengineArgs& a, int nds, int ncu, int nfreqs, const uint32_t* tables, hipStream_t st);
 int fxg_launch_xplain(const XPlainArgs& a, int nprod, int maxchan, hipStream_t st);
 int fxg_launch_xmfma(const XMfmaArgs& a, int ngroup_launch, int group0, const DevXGroup& g, hipStream_t st);
 int fxg_launch_fin(const FinProd* e, int n, int maxout, const float2* acc, float2* res, const UvArgs& uv, hipStream_t st);
