@@ -578,17 +578,30 @@ __global__ void k_fin(const FinProd* e, const float2* acc, float2* res, UvArgs u
 // Baseline weights (core.cpp:1005-1052, 1066-1112) and autocorrelation weights
 // (core.cpp:1306-1370): sequential FP32 sums over the FFTs of the subint.
 
-// One workgroup per entry: a strided partial sum per thread, then a tree over the block.
-__global__ void __launch_bounds__(256) k_fin_weights(const FinWeight* e, const float* w, int B, float* resf) {
-  __shared__ float part[256];
+// One workgroup per entry: a strided partial sum per thread, then a tree over the block.  The time
+// is the latency of the loads (125000 weights took 186 us with 256 threads and one load in flight
+// each), so a thread has eight in flight, and long subints take 1024 threads.
+template <int NTH>
+__global__ void __launch_bounds__(NTH) k_fin_weights(const FinWeight* e, const float* w, int B, float* resf) {
+  __shared__ float part[NTH];
   const FinWeight f = e[blockIdx.x];
   const float* w1 = w + (long long)f.ds1 * B;
   const float* w2 = f.ds2 >= 0 ? w + (long long)f.ds2 * B : nullptr;
   float s = 0.0f;
-  for (int i = threadIdx.x; i < B; i += blockDim.x) s += w2 ? w1[i] * w2[i] : w1[i];
+  for (int i = threadIdx.x; i < B; i += 8 * NTH) {
+    float a[8], b[8];
+#pragma unroll
+    for (int k = 0; k < 8; ++k) {
+      const int at = i + k * NTH;
+      a[k] = at < B ? w1[at] : 0.0f;
+      b[k] = w2 && at < B ? w2[at] : 1.0f;
+    }
+#pragma unroll
+    for (int k = 0; k < 8; ++k) s += a[k] * b[k];
+  }
   part[threadIdx.x] = s;
   __syncthreads();
-  for (int h = 128; h > 0; h >>= 1) {
+  for (int h = NTH / 2; h > 0; h >>= 1) {
     if (threadIdx.x < h) part[threadIdx.x] += part[threadIdx.x + h];
     __syncthreads();
   }
@@ -682,7 +695,8 @@ int fxg_launch_add_at(const int* idx, const float* val, int n, float* resf, hipS
 
 int fxg_launch_fin_weights(const FinWeight* e, int n, const float* w, int B, float* resf, hipStream_t st) {
   if (n == 0) return 0;
-  hipLaunchKernelGGL(k_fin_weights, dim3(n), dim3(256), 0, st, e, w, B, resf);
+  if (B > 8192) hipLaunchKernelGGL(k_fin_weights<1024>, dim3(n), dim3(1024), 0, st, e, w, B, resf);
+  else hipLaunchKernelGGL(k_fin_weights<256>, dim3(n), dim3(256), 0, st, e, w, B, resf);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 

@@ -38,9 +38,10 @@ def test_row_and_fft_edges(gpu, xe, rows, ffts):
     _check(cfg, xe, seed=32)
 
 
-@pytest.mark.parametrize("ffts,chunk", [(700, 0), (700, 264)])
+@pytest.mark.parametrize("ffts,chunk", [(700, 0), (700, 264), (9001, 0)])
 def test_long_runs_and_chunks(gpu, ffts, chunk):
-    """More FFTs than one run of the plain X-engine's sums, in one chunk and in three."""
+    """More FFTs than one run of the plain X-engine's sums, in one chunk and in three, and more
+    than the weight sums take with their smaller workgroup."""
     cfg = cf.standard_config(4, 2, [4800.0], 16.0, 128, subint_ns=ffts * 8000, xengine="fp32", seed=33,
                              chunk_ffts=chunk, max_delay_us=50.0)
     _check(cfg, "fp32", seed=34)
