@@ -1585,6 +1585,7 @@ struct TimedLaunch {
 
 int ntb_for(const fxg_ctx* ctx, int L) {
   if (ctx->fsel.ntb) return ctx->fsel.ntb;
+  if (L == 8192 && ctx->fsel.mat) return 1024;   // no form asked for (see fe_minwaves)
   return L >= 4096 ? 512 : 256;
 }
 

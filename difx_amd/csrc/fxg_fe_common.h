@@ -581,8 +581,9 @@ __device__ void fe_range(const FengineArgs& args, const float2* __restrict__ twi
       // rotator (orders 1, 2) of this thread's samples and fractional-sample phasors of its
       // channels: shared by the bands of the freq, so they can be computed once per freq
       // (FXG_F_HOIST) when a thread holds one butterfly position, at the cost of registers
-      constexpr bool HOIST_ROT = (V == 1) && (FXG_F_HOIST & 1);
-      constexpr bool HOIST = (V == 1) && (FXG_F_HOIST & 2);
+      // (complex data has few bands per freq: the registers are worth more there)
+      constexpr bool HOIST_ROT = (V == 1) && (FXG_F_HOIST & 1) && !(CPLX && L >= 4096);
+      constexpr bool HOIST = (V == 1) && (FXG_F_HOIST & 2) && !(CPLX && L >= 4096);
       constexpr int NKEEP = CPLX ? 8 : 4;
       // Post-F rotation of real data (order 0): the FFT input is real, so two bands of the
       // freq go through one complex FFT as a + ib and are split after it,
@@ -691,14 +692,23 @@ __device__ void fe_range(const FengineArgs& args, const float2* __restrict__ twi
             }
             continue;
           }
+          // complex 8-bit samples: the sixteen loads of a position are issued before any is used
+          // (invalid samples read the buffer's first bytes, if it has any)
+          unsigned br[8], bi[8];
 #pragma unroll
-          for (int s = 0; s < 8; ++s) {             // complex 8-bit samples
-            const float2 rot = HOIST_ROT ? rot_h[s] : rot_l[HOIST_ROT ? 0 : s];
-            float2 x = make_float2(0.f, 0.f);
-            if ((fok[u] >> s) & 1u) {
-              const GBytes pp = data + wv[u][s] + 2 * band;
-              x = make_float2(slut8[pp[0]], slut8[pp[1]]);
+          for (int s = 0; s < 8; ++s) {
+            br[s] = bi[s] = 0u;
+            if (anyload) {
+              const GBytes pp = data + (((fok[u] >> s) & 1u) ? wv[u][s] + 2u * (unsigned)band : 0u);
+              br[s] = pp[0];
+              bi[s] = pp[1];
             }
+          }
+#pragma unroll
+          for (int s = 0; s < 8; ++s) {
+            const float2 rot = HOIST_ROT ? rot_h[s] : rot_l[HOIST_ROT ? 0 : s];
+            const bool ok = (fok[u] >> s) & 1u;
+            const float2 x = make_float2(ok ? slut8[br[s]] : 0.0f, ok ? slut8[bi[s]] : 0.0f);
             v[u][s] = cmul(rot, x);
             // complex LSB: the reference conj-flips the spectrum (mode.cpp:1186-1201);
             // FFT(conj y)[c] = conj(FFT(y)[-c]) gives the same channels without a flip

@@ -38,13 +38,18 @@ __global__ void k_fftparams(FengineArgs args) {
   args.params[(long long)d * args.chunkcap + lt] = fd;
 }
 
-#ifndef FXG_F_MINWAVES
-#define FXG_F_MINWAVES 1
-#endif
+// Waves per SIMD the register allocation is held to.  A 4096-point FFT on 512 threads takes 2 of
+// them and half of a CU's LDS: held to 4 (128 registers, real data would take 130, complex 145) a
+// CU runs two workgroups, so that one works while the other waits at a barrier: 4.95 -> 3.54 ms for
+// 16 stations' real 2-bit samples at 256 MHz in 0.5 s, 9.35 -> 6.34 ms for 64 stations' complex
+// 8-bit samples at 16 MHz in 1 s (with the byte loads of fe_range issued together).  An 8192-point
+// FFT takes a CU's LDS by itself: 1024 threads with one butterfly position each give it 4 waves
+// per SIMD: 1.75 -> 1.61 ms for 8 stations x 8 bands, 1000 FFTs.
+constexpr int fe_minwaves(int L, int NTB) { return (L == 4096 && NTB == 512) || NTB == 1024 ? 4 : 1; }
 
 // One FFT length: workgroup (x, y) = units [x*units_per_wg, ...) of datastream dslist[y].
 template <int L, bool CPLX, int ORDER, int NTB>
-__global__ void __launch_bounds__(NTB, FXG_F_MINWAVES) k_fengine(FengineArgs args) {
+__global__ void __launch_bounds__(NTB, fe_minwaves(L, NTB)) k_fengine(FengineArgs args) {
   extern __shared__ float2 fx_smem[];
   const int d = args.dslist[blockIdx.y];
   const int nunits = args.nffts_pad / 8;
@@ -247,6 +252,8 @@ static int launch_len(const FengineArgs& a, int L, int nds, hipStream_t st) {
 }
 
 int fxg_launch_fengine(const FengineArgs& a, int L, int iscomplex, int nds, int ntb, hipStream_t st) {
+  if (ntb == 1024)                            // 8192-point FFTs only
+    return L != 8192 ? -2 : iscomplex ? launch_f<8192, true, 1024>(a, nds, st) : launch_f<8192, false, 1024>(a, nds, st);
   if (ntb == 512) return iscomplex ? launch_len<true, 512>(a, L, nds, st) : launch_len<false, 512>(a, L, nds, st);
   if (ntb == 256) return iscomplex ? launch_len<true, 256>(a, L, nds, st) : launch_len<false, 256>(a, L, nds, st);
   if (ntb == 128) return iscomplex ? launch_len<true, 128>(a, L, nds, st) : launch_len<false, 128>(a, L, nds, st);
