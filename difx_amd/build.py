@@ -18,7 +18,7 @@ HERE = Path(__file__).resolve().parent
 CSRC = HERE / "csrc"
 INCLUDE = HERE.parent / "include"
 LIB = HERE / "libfxg.so"
-SOURCES = ["fxg_fengine.hip", "fxg_fpersist.hip", "fxg_fbig.hip", "fxg_fmat.hip", "fxg_xengine.hip", "fxg_api.cpp",
+SOURCES = ["fxg_fengine.hip", "fxg_fpersist.hip", "fxg_fbig.hip", "fxg_freg.hip", "fxg_fmat.hip", "fxg_xengine.hip", "fxg_api.cpp",
            "fxg_server.cpp", "fxg_vdifmux.hip", "fxg_control.cpp",
            "fxg_visnorm.hip", "fxg_kurt.hip", "fxg_pcal.hip"]
 ARCH = "gfx950"

@@ -106,6 +106,8 @@ struct fxg_ctx {
     long long twL_off = 0;       // big: exp(-2 pi i j / L), j < L
     int wgx = 1;                 // big: workgroups per datastream (scratch rows)
     bool mat = false;            // the matrix F-engine takes it (see build_tables)
+    bool reg = false;            // the register F-engine takes it
+    long long twr_off = 0;       // its twiddles in d_twiddle
   };
   float2* d_bigscratch = nullptr;
   int bigL = 0;
@@ -116,7 +118,7 @@ struct fxg_ctx {
     int mode = FXG_F_PER_LENGTH;
     int ntb = 0;                 // workgroup size; 0 = 256 below L = 4096, 512 from there
     int grid_mult = 1;           // persistent: workgroups per CU
-    bool mat = false;            // the matrix F-engine where it applies
+    bool mat = false;            // the matrix and the register F-engine where they apply
   };
   uint32_t* d_fmat = nullptr;    // its constant tables
   FChoice fsel;
@@ -976,6 +978,8 @@ int build_tables(fxg_ctx* ctx) {
     c.mat = c.L == 2048 && !c.cplx && ctx->rotorder != 2;
     for (int d : c.dsl) c.mat = c.mat && ctx->h_ds[d].nbits == 2;
     anymat = anymat || c.mat;
+    c.reg = !c.cplx;               // the register F-engine: long FFTs of 2-bit samples
+    for (int d : c.dsl) c.reg = c.reg && ctx->h_ds[d].nbits == 2 && fxg_freg_takes(c.L, ctx->rotorder, ctx->h_ds[d].S, c.phcap);
   }
   if (anymat) {
     static const std::vector<uint32_t> t = [] {   // the same for every context
@@ -1001,6 +1005,11 @@ int build_tables(fxg_ctx* ctx) {
           const double a = -TWO_PI * (double)j / (double)c.L;
           tw.push_back(make_float2((float)std::cos(a), (float)std::sin(a)));
         }
+      }
+      if (c.reg) {
+        c.twr_off = (long long)tw.size();
+        const std::vector<float2>& t = fxg_freg_tables(c.L);
+        tw.insert(tw.end(), t.begin(), t.end());
       }
       const int Lt = c.big ? 2048 : c.L;
       if (tw_of_L.count(Lt)) { c.tw_off = tw_of_L[Lt]; continue; }
@@ -1818,10 +1827,16 @@ int build_items(fxg_ctx* ctx) {
 int launch_fengines(fxg_ctx* ctx, FengineArgs& fa, hipStream_t st) {
   const int nunits = fa.nffts_pad / 8;
   for (const auto& fc : ctx->fclasses) {
-    if (!fc.big || ctx->fsel.mode == FXG_F_PERSISTENT) continue;
+    const bool reg = ctx->fsel.mat && fc.reg;
+    if ((!fc.big && !reg) || ctx->fsel.mode == FXG_F_PERSISTENT) continue;
     fa.twiddle = ctx->d_twiddle + fc.tw_off;
     fa.dslist = ctx->d_dslist + fc.dsl_off;
     fa.phcap = fc.phcap;
+    if (reg) {
+      if (fxg_launch_freg(fa, fc.L, (int)fc.dsl.size(), ctx->ncu, ctx->d_twiddle + fc.twr_off, st))
+        return fail(ctx, FXG_E_HIP, "F-engine launch");
+      continue;
+    }
     if (fxg_launch_fbig(fa, fc.L, fc.cplx, (int)fc.dsl.size(), fc.wgx, ctx->d_bigscratch,
                         ctx->d_twiddle + fc.twL_off, st))
       return fail(ctx, FXG_E_HIP, "four-step F-engine launch");
@@ -1858,7 +1873,7 @@ int launch_fengines(fxg_ctx* ctx, FengineArgs& fa, hipStream_t st) {
     return FXG_OK;
   }
   for (const auto& fc : ctx->fclasses) {
-    if (fc.big) continue;
+    if (fc.big || (ctx->fsel.mat && fc.reg)) continue;
     const int ncl = (int)fc.dsl.size();
     if (ctx->fsel.mat && fc.mat) {
       fa.dslist = ctx->d_dslist + fc.dsl_off;
@@ -2146,8 +2161,8 @@ int autotune(fxg_ctx* ctx) {
     cand.emplace_back(name, c);
   };
   for (const auto& fc : ctx->fclasses)
-    if (fc.mat && ctx->cfg_fmode == FXG_F_AUTO && !ctx->cfg_fthreads) {
-      add("matrix where it applies, else per-length, 256/512 threads by length", FXG_F_PER_LENGTH, 0, 1);
+    if ((fc.mat || fc.reg) && ctx->cfg_fmode == FXG_F_AUTO && !ctx->cfg_fthreads) {
+      add("matrix or register kernel where they apply, else per-length, 256/512 threads by length", FXG_F_PER_LENGTH, 0, 1);
       cand.back().second.mat = true;
       break;
     }
@@ -3299,7 +3314,7 @@ int fxg_delay_interpolator(fxg_ctx* ctx, int32_t ds, int32_t sec, int32_t ns, do
 int fxg_autotune_report(const fxg_ctx* ctx, char* buf, int32_t len) {
   if (!ctx || !buf || len < 1) return FXG_E_INVALID;
   std::string r = "F-engine: ";
-  r += ctx->fsel.mode == FXG_F_PERSISTENT ? "persistent" : ctx->fsel.mat ? "matrix where it applies, else per-length" : "per-length";
+  r += ctx->fsel.mode == FXG_F_PERSISTENT ? "persistent" : ctx->fsel.mat ? "matrix or register kernel where they apply, else per-length" : "per-length";
   r += ", threads " + (ctx->fsel.ntb ? std::to_string(ctx->fsel.ntb) : std::string("by length"));
   if (ctx->fsel.mode == FXG_F_PERSISTENT) r += ", " + std::to_string(ctx->fsel.grid_mult) + " workgroup(s)/CU";
   for (const auto& e : ctx->tune_log) {

@@ -1,6 +1,7 @@
 // Internal tables shared by the host layer and the device kernels of libfxg.
 #pragma once
 #include <hip/hip_runtime.h>
+#include <vector>
 #include <stdint.h>
 #include "../../include/fxg.h"
 
@@ -322,6 +323,11 @@ size_t fxg_fengine_lds(int L, int ntb, int phcap, int order);
 int fxg_launch_fbig(const FengineArgs& a, int L, int iscomplex, int nds, int wgx, float2* scratch,
                     const float2* twL, hipStream_t st);
 size_t fxg_fbig_lds(int ntb, int phcap);
+
+// Register F-engine (fxg_freg.hip): long FFTs of real 2-bit samples.
+bool fxg_freg_takes(int L, int order, int S, int phcap);
+const std::vector<float2>& fxg_freg_tables(int L);
+int fxg_launch_freg(const FengineArgs& a, int L, int nds, int ncu, const float2* tw, hipStream_t st);
 // Matrix F-engine (fxg_fmat.hip): words of its constant tables and their three parts.
 constexpr int FMAT_W_WORDS = 2 * 4 * 2 * 64 * 4;
 constexpr int FMAT_T_WORDS = 2 * 16 * 64 * 2;
