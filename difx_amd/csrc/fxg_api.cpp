@@ -978,8 +978,9 @@ int build_tables(fxg_ctx* ctx) {
     c.mat = c.L == 2048 && !c.cplx && ctx->rotorder != 2;
     for (int d : c.dsl) c.mat = c.mat && ctx->h_ds[d].nbits == 2;
     anymat = anymat || c.mat;
-    c.reg = !c.cplx;               // the register F-engine: long FFTs of 2-bit samples
-    for (int d : c.dsl) c.reg = c.reg && ctx->h_ds[d].nbits == 2 && fxg_freg_takes(c.L, ctx->rotorder, ctx->h_ds[d].S, c.phcap);
+    c.reg = true;                  // the register F-engine: long FFTs
+    for (int d : c.dsl)
+      c.reg = c.reg && fxg_freg_takes(c.L, c.cplx, ctx->h_ds[d].nbits, ctx->rotorder, ctx->h_ds[d].S, c.phcap);
   }
   if (anymat) {
     static const std::vector<uint32_t> t = [] {   // the same for every context
@@ -1833,7 +1834,7 @@ int launch_fengines(fxg_ctx* ctx, FengineArgs& fa, hipStream_t st) {
     fa.dslist = ctx->d_dslist + fc.dsl_off;
     fa.phcap = fc.phcap;
     if (reg) {
-      if (fxg_launch_freg(fa, fc.L, (int)fc.dsl.size(), ctx->ncu, ctx->d_twiddle + fc.twr_off, st))
+      if (fxg_launch_freg(fa, fc.L, fc.cplx, (int)fc.dsl.size(), ctx->ncu, ctx->d_twiddle + fc.twr_off, st))
         return fail(ctx, FXG_E_HIP, "F-engine launch");
       continue;
     }

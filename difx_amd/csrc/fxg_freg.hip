@@ -1,6 +1,6 @@
-// F-engine for long FFTs of real 2-bit samples (8192 to 32768 points) with the whole FFT in the
-// registers of one workgroup.  What one FFT computes is what the fused F-engine computes
-// (Mode::process, mode.cpp:634-1374: decode, rotator, L-point FFT, channel selection,
+// F-engine for long FFTs (4096 to 32768 points) of real 2-bit and complex 8-bit samples with the
+// whole FFT in the registers of one workgroup.  What one FFT computes is what the fused F-engine
+// computes (Mode::process, mode.cpp:634-1374: decode, rotator, L-point FFT, channel selection,
 // fractional-sample correction).
 //
 // L/32 threads hold 32 points each and run three Stockham passes of radix 32, 32 and L/1024; the
@@ -11,7 +11,8 @@
 // points, 76 % of the cycles (the four-step kernel: 118, 65 %; it also wrote and read each
 // spectrum once in L2 and MALL).  Measured, 16 stations, 1001 FFTs of 32768 points in 8 bands
 // and 1001 of 16384 in 8: 22.1 -> 12.0 ms and 9.0 -> 4.5 ms; 8 stations, 1000 FFTs of 8192 points
-// in 8 bands (k_fengine before): 1.61 -> 1.19 ms.
+// in 8 bands (k_fengine before): 1.61 -> 1.19 ms; 16 stations, 4096 points in 16 bands 3.5 -> 2.6 ms;
+// 64 stations of complex 8-bit samples, 3906 FFTs of 4096 points: 6.3 -> 3.6 ms.
 #include "fxg_fe_common.h"
 #include <algorithm>
 #include <cmath>
@@ -113,6 +114,7 @@ __device__ __forceinline__ int opaque(int t) {
   asm volatile("" : "+v"(t));
   return t;
 }
+typedef const __attribute__((address_space(1))) uint16_t* GHalfs;
 __device__ __forceinline__ void fence() { __builtin_amdgcn_sched_barrier(0); }
 
 // An FFT's parameters, uniform: read by scalar loads where they are used.
@@ -129,45 +131,49 @@ struct RPlan {
   static constexpr int NT = L / 32;               // threads of an FFT
   static constexpr int R = L / 1024;              // radix of the last pass
   static constexpr int NB = 32 / R;               // its butterflies per thread
+  static constexpr int G = L == 4096 ? 2 : 1;     // FFTs side by side in a workgroup
   static constexpr int TW1 = 31 * 32;             // twiddles of the second pass, [s - 1][k]
   static constexpr int TW2 = (R - 1) * 1024;      // and of the last, [s - 1][j]
   // register of X[t + q NT] after the last pass: butterfly q % NB, output q / NB
   static constexpr int reg(int q) {
     const int b = q % NB, r = q / NB;
-    return R == 32 ? reg32(r) : R == 16 ? b * 16 + 4 * (r & 3) + (r >> 2) : b * 8 + r;
+    return R == 32 ? reg32(r) : R == 16 ? b * 16 + 4 * (r & 3) + (r >> 2) : b * R + r;
   }
 };
 
 template <int L>
-size_t freg_lds_bytes(int phcap) {
-  return sizeof(float) * (size_t)L + sizeof(float2) * ((size_t)RPlan<L>::TW1 + 2 * (size_t)phcap) +
-         sizeof(float) * ((size_t)phcap + 8) + stage_lds_bytes(phcap);
+size_t freg_lds_bytes(int cplx, int order, int phcap) {
+  constexpr int G = RPlan<L>::G;
+  return sizeof(float) * (size_t)L * G + sizeof(float2) * ((size_t)RPlan<L>::TW1 + 2 * (size_t)G * phcap) +
+         sizeof(float) * ((order == 2 ? (size_t)G * phcap : 0) + (cplx ? 256 : 8)) + stage_lds_bytes(phcap);
 }
 
 }  // namespace
 
 // Workgroup (x, y): FFTs [x * upw, ...) of datastream dslist[y], consecutive ones so that their
 // 16-bit spectra complete each other's lines in one L2.  128 registers: at 32768
-// points one workgroup of 16 waves per CU, at 16384 two of 8 and at 8192 three of 4 (by LDS), so that
-// one works while the others wait.
-template <int L, int ORDER>
-__global__ void __launch_bounds__(L / 32, 4) k_freg(FengineArgs args, const float2* __restrict__ tw, int upw) {
+// points one workgroup of 16 waves per CU, at 16384 two of 8, below three of 4 (by LDS; 4096
+// points two FFTs side by side), so that one works while the others wait.
+template <int L, bool CPLX, int ORDER>
+__global__ void __launch_bounds__(L / 32 * RPlan<L>::G, 4) k_freg(FengineArgs args, const float2* __restrict__ tw, int upw) {
   using P = RPlan<L>;
-  constexpr int NT = P::NT;
+  constexpr int NT = P::NT, G = P::G, NTB = NT * G;
   extern __shared__ float2 fx_smem[];
+  const int tid = threadIdx.x;
+  const int g = G == 1 ? 0 : __builtin_amdgcn_readfirstlane(tid / NT), t0 = tid - g * NT;
+  const int ph = args.phcap;
   float2* stw = fx_smem;                          // twiddles of the second pass
-  float2* srot = stw + P::TW1;
-  float2* sfrac = srot + args.phcap;
-  float* xb = reinterpret_cast<float*>(sfrac + args.phcap);    // exchange buffer
-  float* squad = xb + L;
-  float* slev = squad + args.phcap;               // the format's four levels
-  float* scf = slev + 8;                          // staged channel-frequency tables
-  const int t0 = threadIdx.x;
+  float2* srot = stw + P::TW1 + g * ph;
+  float2* sfrac = stw + P::TW1 + (G + g) * ph;
+  float* xb = reinterpret_cast<float*>(stw + P::TW1 + 2 * G * ph) + g * L;    // exchange buffer
+  float* squad = reinterpret_cast<float*>(stw + P::TW1 + 2 * G * ph) + G * L + g * ph;
+  float* slev = reinterpret_cast<float*>(stw + P::TW1 + 2 * G * ph) + G * (ORDER == 2 ? L + ph : L);   // the sample levels
+  float* scf = slev + (CPLX ? 256 : 8);                        // staged channel-frequency tables
   const int d = args.dslist[blockIdx.y];
   const CDevDs dsp = (CDevDs)(args.ds + d);
-  for (int m = t0; m < P::TW1; m += NT) stw[m] = tw[m];
-  if (t0 < 4) slev[t0] = lut2(dsp->format, t0);
-  stage_cf(args, dsp, scf, t0, NT);
+  for (int m = tid; m < P::TW1; m += NTB) stw[m] = tw[m];
+  for (int m = tid; m < (CPLX ? 256 : 4); m += NTB) slev[m] = CPLX ? lut8(m) : lut2(dsp->format, m);
+  stage_cf(args, dsp, scf, tid, NTB);
   const float2* __restrict__ tw2 = tw + P::TW1;
   DsConst k;
   k.C = dsp->C; k.S = dsp->S; k.NS = dsp->NS; k.NFS = dsp->NFS; k.nrec = dsp->nrecbands;
@@ -186,7 +192,8 @@ __global__ void __launch_bounds__(L / 32, 4) k_freg(FengineArgs args, const floa
   const int cap = args.chunkcap;
 
   const int lt0 = blockIdx.x * upw, lt1 = min(lt0 + upw, args.nffts_pad);
-  for (int lt = lt0; lt < lt1; ++lt) {
+  for (int lb = lt0; lb < lt1; lb += G) {          // (lt1 - lt0 is a multiple of G)
+    const int lt = lb + g;
     const int n0 = params[lt].n0;
     const bool fok_all = params[lt].ok != 0;       // flagged FFTs: zero spectra (mode.cpp:656-669)
     const bool whole = fok_all && params[lt].weight == 1.0f;   // every sample of the window decodes
@@ -199,7 +206,7 @@ __global__ void __launch_bounds__(L / 32, 4) k_freg(FengineArgs args, const floa
       const FreqConst rf = load_freq(dsp->rf[f]);
       const FftDelay fd = load_delay(params[lt]);
       if (ORDER != 0) build_rotator<ORDER>(srot, squad, k, rf, fd, L, t0, NT);
-      build_frac<ORDER>(sfrac, k, rf, 0, scf, fd, dsp->rf[f].bhd[0], make_float2(dsp->rf[f].pcre[0], dsp->rf[f].pcim[0]), t0, NT);
+      build_frac<ORDER>(sfrac, k, rf, CPLX, scf, fd, dsp->rf[f].bhd[0], make_float2(dsp->rf[f].pcre[0], dsp->rf[f].pcim[0]), t0, NT);
       }
       __syncthreads();
       uint32_t pk[2][2], okm = ~0u;
@@ -209,11 +216,11 @@ __global__ void __launch_bounds__(L / 32, 4) k_freg(FengineArgs args, const floa
           __syncthreads();                        // the previous band's phasor reads are done
           const FreqConst rf = load_freq(dsp->rf[f]);
           const FftDelay fd = load_delay(params[lt]);
-          build_frac<ORDER>(sfrac, k, rf, 0, scf, fd, dsp->rf[f].bhd[kb], make_float2(dsp->rf[f].pcre[kb], dsp->rf[f].pcim[kb]), t0, NT);
+          build_frac<ORDER>(sfrac, k, rf, CPLX, scf, fd, dsp->rf[f].bhd[kb], make_float2(dsp->rf[f].pcre[kb], dsp->rf[f].pcim[kb]), t0, NT);
         }
         // The 2-bit fields of this thread's samples n = t + s NT, for two bands at a time: a
         // sample word holds every band's field.
-        if ((kb & 1) == 0) {
+        if (!CPLX && (kb & 1) == 0) {
           const int t = opaque(t0);
           const int sh0 = 2 * band, sh1 = 2 * (kb + 1 < nbands ? dsp->rf[f].band[kb + 1] : band);
           pk[0][0] = pk[0][1] = pk[1][0] = pk[1][1] = 0u;
@@ -277,8 +284,38 @@ __global__ void __launch_bounds__(L / 32, 4) k_freg(FengineArgs args, const floa
           }
         }
         float2 v[32];
+        const bool lsb = dsp->rf[f].lsb != 0;
         const uint32_t p0 = kb & 1 ? pk[1][0] : pk[0][0], p1 = kb & 1 ? pk[1][1] : pk[0][1];
         fence();
+        if (CPLX) {
+          // complex 8-bit samples: both bytes in one load, sixteen in flight; an invalid sample
+          // reads the buffer's first bytes, if it has any
+          const int t = opaque(t0);
+          const unsigned g0 = (unsigned)n0 + (unsigned)t;
+          const bool any = fok_all && nframes > 0;
+          okm = whole ? ~0u : 0u;
+#pragma unroll
+          for (int sb = 0; sb < 32; sb += 16) {
+            unsigned w[16];
+#pragma unroll
+            for (int s = 0; s < 16; ++s) {
+              const unsigned gs = g0 + (unsigned)((sb + s) * NT);
+              unsigned fr = (unsigned)((double)gs * inv_spf);
+              unsigned within = gs - fr * (unsigned)k.spf;
+              if (within >= (unsigned)k.spf) { within -= k.spf; ++fr; }
+              bool ok = whole;
+              if (!whole) {
+                ok = any && fr < (unsigned)nframes && sample_ok(fv[fr], fz, fr, within);
+                okm |= (ok ? 1u : 0u) << (sb + s);
+              }
+              const unsigned at = fr * (unsigned)k.framebytes + (unsigned)k.headerbytes + (within * (unsigned)k.nrec + band) * 2u;
+              w[s] = any ? *(GHalfs)(data + (ok ? at : 0u)) : 0u;
+            }
+#pragma unroll
+            for (int s = 0; s < 16; ++s) v[sb + s] = make_float2(slev[w[s] & 255u], slev[w[s] >> 8]);
+            fence();
+          }
+        }
         {
           const int t = opaque(t0);
           const float2 sub = ORDER != 0 ? srot[t & (S - 1)] : make_float2(1.0f, 0.0f);
@@ -294,14 +331,16 @@ __global__ void __launch_bounds__(L / 32, 4) k_freg(FengineArgs args, const floa
           const float2* __restrict__ step = srot + S + t / S;    // NT is a multiple of S
 #pragma unroll
           for (int s = 0; s < 32; ++s) {
-            const float x = slev[((s < 16 ? p0 : p1) >> (2 * (s & 15))) & 3u];
+            const float x = CPLX ? 0.0f : slev[((s < 16 ? p0 : p1) >> (2 * (s & 15))) & 3u];
             if (ORDER == 0) {
               v[s] = make_float2(x, 0.0f);
             } else {
               float2 rot = sub;
               if (ORDER == 2) { rot = cmul(sub, qpow); qpow = cmul(qpow, qstep); }
               rot = cmul(rot, step[s * (NT / S)]);
-              v[s] = make_float2(x * rot.x, x * rot.y);
+              v[s] = CPLX ? cmul(rot, v[s]) : make_float2(x * rot.x, x * rot.y);
+              // complex LSB: conj input gives the conjugate-flipped spectrum (mode.cpp:1186-1201)
+              if (CPLX && lsb) v[s].y = -v[s].y;
             }
             if (s % 8 == 7) fence();
           }
@@ -324,13 +363,13 @@ __global__ void __launch_bounds__(L / 32, 4) k_freg(FengineArgs args, const floa
           for (int i = 0; i < 8; ++i) xw[i ^ (t & 7)] = make_float4(v[i].x, v[8 + i].x, v[16 + i].x, v[24 + i].x);
           __syncthreads();
 #pragma unroll
-          for (int s = 0; s < 32; ++s) v[s].x = xb[rd + s * NT];
+          for (int s = 0; s < 32; ++s) v[s].x = xb[(NT == 128 && (s & 1) ? rd ^ 16 : rd) + s * NT];
           __syncthreads();
 #pragma unroll
           for (int i = 0; i < 8; ++i) xw[i ^ (t & 7)] = make_float4(v[i].y, v[8 + i].y, v[16 + i].y, v[24 + i].y);
           __syncthreads();
 #pragma unroll
-          for (int s = 0; s < 32; ++s) v[s].y = xb[rd + s * NT];
+          for (int s = 0; s < 32; ++s) v[s].y = xb[(NT == 128 && (s & 1) ? rd ^ 16 : rd) + s * NT];
         }
         // ---- pass 2
         {
@@ -377,14 +416,18 @@ __global__ void __launch_bounds__(L / 32, 4) k_freg(FengineArgs args, const floa
 #pragma unroll
             for (int s = 0; s < 8; ++s)
               if (s0 + s < P::R) z[b * P::R + s0 + s] = cmul(v[b + (s0 + s) * P::NB], w[s]);
-            fence();
+            if (P::R > 4 || (b & 1)) fence();
           }
           if (P::R == 32) dft32(z);
           else if (P::R == 16) dft16p(z + b * P::R);
-          else dft8k<0>(z + b * P::R);
+          else if (P::R == 8) dft8k<0>(z + b * P::R);
+          else dft4k<0>(z + b * P::R);
         }
-        // ---- the kept half of the channels c = t + m NT (USB X[c], LSB X[C + c], mode.cpp:1205),
-        // times the fractional-sample phasor and the output scale
+        // ---- the kept channels c = t + m NT, times the fractional-sample phasor and the output
+        // scale: real USB X[c], LSB X[C + c] (mode.cpp:1205); complex all, halves swapped for double
+        // sideband (mode.cpp:1191-1192, 1211-1213)
+        constexpr int KEEP = CPLX ? 32 : 16;
+        if (CPLX && lsb && !k.dsb && t == 0) z[P::reg(0)].y = -z[P::reg(0)].y;   // DC is not flipped (mode.cpp:1199-1200)
         const float2 fsub0 = sfrac[t & (S - 1)];
         const float2 fsub = make_float2(fsub0.x * fs, fsub0.y * fs);
         const float2* __restrict__ fstep = sfrac + S + t / S;
@@ -393,7 +436,7 @@ __global__ void __launch_bounds__(L / 32, 4) k_freg(FengineArgs args, const floa
           if (args.out_mode == 0) {
             float2* __restrict__ o32 = args.spec32 + dsp->spec_off + ((long long)band * cap + lt) * k.C;
 #pragma unroll
-            for (int m = 0; m < 16; ++m) (o32 + m * NT)[(unsigned)t] = cmul(z[P::reg(H + m)], cmul(fsub, fstep[m * (NT / S)]));
+            for (int m = 0; m < KEEP; ++m) (o32 + m * NT)[(unsigned)t] = cmul(z[P::reg((H + m) & 31)], cmul(fsub, fstep[m * (NT / S)]));
             return;
           }
           auto store16 = [&](auto mode_c) {
@@ -409,10 +452,10 @@ __global__ void __launch_bounds__(L / 32, 4) k_freg(FengineArgs args, const floa
             const long long cs16 = ((long long)(NT >> twl) * cap) << twl;
             const bool zoom = dsp->nzout > 0;
 #pragma unroll
-            for (int m = 0; m < 16; ++m) {
-              const uint32_t o = pack16m<OM>(cmul(z[P::reg(H + m)], cmul(fsub, fstep[m * (NT / S)])));
+            for (int m = 0; m < KEEP; ++m) {
+              const uint32_t o = pack16m<OM>(cmul(z[P::reg((H + m) & 31)], cmul(fsub, fstep[m * (NT / S)])));
               (o16 + m * cs16)[ot] = o;
-              if (zoom) z[P::reg(H + m)].x = __uint_as_float(o);   // kept for the windows
+              if (zoom) z[P::reg((H + m) & 31)].x = __uint_as_float(o);   // kept for the windows
             }
             // zoom windows of this band: the same channels again, as rows of the zoom freq's group
             for (int zz = 0; zz < dsp->nzout; ++zz) {
@@ -423,16 +466,16 @@ __global__ void __launch_bounds__(L / 32, 4) k_freg(FengineArgs args, const floa
               uint32_t* __restrict__ oz = args.spec16 + zg->spec_off + (long long)dsp->zout_row[zz] * zg->rowstride +
                                           ((long long)lt << zl);
 #pragma unroll
-              for (int m = 0; m < 16; ++m) {
+              for (int m = 0; m < KEEP; ++m) {
                 const int cz = t + m * NT - c0;
-                if (cz >= 0 && cz < nz) oz[(((long long)(cz >> zl) * cap) << zl) + (cz & zm)] = __float_as_uint(z[P::reg(H + m)].x);
+                if (cz >= 0 && cz < nz) oz[(((long long)(cz >> zl) * cap) << zl) + (cz & zm)] = __float_as_uint(z[P::reg((H + m) & 31)].x);
               }
             }
           };
           if (args.out_mode == 1) store16(IntC<1>());
           else store16(IntC<2>());
         };
-        if (dsp->rf[f].lsb) emit(IntC<16>());
+        if (CPLX ? k.dsb != 0 : lsb) emit(IntC<16>());
         else emit(IntC<0>());
       }
     }
@@ -441,38 +484,43 @@ __global__ void __launch_bounds__(L / 32, 4) k_freg(FengineArgs args, const floa
 
 namespace {
 
-template <int L, int ORDER>
+template <int L, bool CPLX, int ORDER>
 int launch(const FengineArgs& a, int nds, int ncu, const float2* tw, hipStream_t st) {
   static size_t raised = 0;
-  const size_t lds = freg_lds_bytes<L>(a.phcap);
-  if (raise_lds(k_freg<L, ORDER>, lds, &raised)) return -1;
-  // four rounds of workgroups or more where there are that many FFTs, up to eight FFTs each
-  const long long total = (long long)a.nffts_pad * nds, wgs = 4LL * ncu * (32768 / L);
-  const int upw = (int)std::max(1LL, std::min(8LL, total / wgs));
-  hipLaunchKernelGGL((k_freg<L, ORDER>), dim3((a.nffts_pad + upw - 1) / upw, nds), dim3(L / 32), lds, st, a, tw, upw);
+  constexpr int G = RPlan<L>::G;
+  const size_t lds = freg_lds_bytes<L>(CPLX, ORDER, a.phcap);
+  if (raise_lds(k_freg<L, CPLX, ORDER>, lds, &raised)) return -1;
+  // four rounds of workgroups or more where there are that many FFTs, up to eight FFTs each per
+  // group of threads
+  const long long total = (long long)a.nffts_pad / G * nds, wgs = 4LL * ncu * (32768 / (L * G));
+  const int upw = G * (int)std::max(1LL, std::min(8LL, total / wgs));
+  hipLaunchKernelGGL((k_freg<L, CPLX, ORDER>), dim3((a.nffts_pad + upw - 1) / upw, nds), dim3(L / 32 * G), lds, st, a, tw, upw);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
 template <int L>
-int launch_o(const FengineArgs& a, int nds, int ncu, const float2* tw, hipStream_t st) {
+int launch_o(const FengineArgs& a, int cplx, int nds, int ncu, const float2* tw, hipStream_t st) {
   switch (a.rotorder) {
-    case 0: return launch<L, 0>(a, nds, ncu, tw, st);
-    case 1: return launch<L, 1>(a, nds, ncu, tw, st);
-    case 2: return launch<L, 2>(a, nds, ncu, tw, st);
+    case 0: return cplx || L <= 8192 ? -2 : launch<(L <= 8192 ? 16384 : L), false, 0>(a, nds, ncu, tw, st);
+    case 1: return cplx ? launch<L, true, 1>(a, nds, ncu, tw, st) : launch<L, false, 1>(a, nds, ncu, tw, st);
+    case 2: return cplx ? launch<L, true, 2>(a, nds, ncu, tw, st) : launch<L, false, 2>(a, nds, ncu, tw, st);
   }
   return -2;
 }
 
 }  // namespace
 
-// Whether it takes FFTs of L points of real 2-bit samples: phasor tables (phcap entries, sub-phasors
-// of S) that leave room in LDS for one, two or three workgroups per CU, and S dividing the stride
-// of a thread's samples.  8192 points of post-F rotation (order 0) stay with k_fengine, which puts
-// two bands through one FFT there.
-bool fxg_freg_takes(int L, int order, int S, int phcap) {
-  if (L == 8192 && order == 0) return false;
-  if (L != 8192 && L != 16384 && L != 32768) return false;
-  const size_t lds = L == 32768 ? freg_lds_bytes<32768>(phcap) : L == 16384 ? freg_lds_bytes<16384>(phcap) : freg_lds_bytes<8192>(phcap);
+// Whether it takes FFTs of L points: phasor tables (phcap entries, sub-phasors of S) that leave room
+// in LDS for one, two or three workgroups per CU (fewer would not cover each other's barriers), and S
+// dividing the stride of a thread's samples.  Up to 8192 points of post-F rotation (order 0) stay
+// with k_fengine, which puts two bands through one FFT there.
+bool fxg_freg_takes(int L, int cplx, int nbits, int order, int S, int phcap) {
+  if (nbits != (cplx ? 8 : 2) || (order == 0 && (cplx || L <= 8192))) return false;
+  const size_t lds = L == 32768   ? freg_lds_bytes<32768>(cplx, order, phcap)
+                     : L == 16384 ? freg_lds_bytes<16384>(cplx, order, phcap)
+                     : L == 8192  ? freg_lds_bytes<8192>(cplx, order, phcap)
+                     : L == 4096  ? freg_lds_bytes<4096>(cplx, order, phcap)
+                                  : ~(size_t)0;
   return (L / 32) % S == 0 && (S & (S - 1)) == 0 && lds <= (L == 32768 ? 160u : L == 16384 ? 80u : 53u) * 1024u;
 }
 
@@ -495,11 +543,16 @@ static const std::vector<float2>& tables() {
   return t;
 }
 const std::vector<float2>& fxg_freg_tables(int L) {
-  return L == 32768 ? tables<32768>() : L == 16384 ? tables<16384>() : tables<8192>();
+  return L == 32768 ? tables<32768>() : L == 16384 ? tables<16384>() : L == 8192 ? tables<8192>() : tables<4096>();
 }
 
-int fxg_launch_freg(const FengineArgs& a, int L, int nds, int ncu, const float2* tw, hipStream_t st) {
+int fxg_launch_freg(const FengineArgs& a, int L, int cplx, int nds, int ncu, const float2* tw, hipStream_t st) {
   if (fxg_launch_fftparams(a, nds, st)) return -1;
-  return L == 32768 ? launch_o<32768>(a, nds, ncu, tw, st) : L == 16384 ? launch_o<16384>(a, nds, ncu, tw, st)
-                                                     : L == 8192 ? launch_o<8192>(a, nds, ncu, tw, st) : -2;
+  switch (L) {
+    case 4096: return launch_o<4096>(a, cplx, nds, ncu, tw, st);
+    case 8192: return launch_o<8192>(a, cplx, nds, ncu, tw, st);
+    case 16384: return launch_o<16384>(a, cplx, nds, ncu, tw, st);
+    case 32768: return launch_o<32768>(a, cplx, nds, ncu, tw, st);
+  }
+  return -2;
 }

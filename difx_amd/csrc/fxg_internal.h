@@ -325,9 +325,9 @@ int fxg_launch_fbig(const FengineArgs& a, int L, int iscomplex, int nds, int wgx
 size_t fxg_fbig_lds(int ntb, int phcap);
 
 // Register F-engine (fxg_freg.hip): long FFTs of real 2-bit samples.
-bool fxg_freg_takes(int L, int order, int S, int phcap);
+bool fxg_freg_takes(int L, int cplx, int nbits, int order, int S, int phcap);
 const std::vector<float2>& fxg_freg_tables(int L);
-int fxg_launch_freg(const FengineArgs& a, int L, int nds, int ncu, const float2* tw, hipStream_t st);
+int fxg_launch_freg(const FengineArgs& a, int L, int cplx, int nds, int ncu, const float2* tw, hipStream_t st);
 // Matrix F-engine (fxg_fmat.hip): words of its constant tables and their three parts.
 constexpr int FMAT_W_WORDS = 2 * 4 * 2 * 64 * 4;
 constexpr int FMAT_T_WORDS = 2 * 16 * 64 * 2;

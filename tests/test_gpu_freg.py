@@ -1,4 +1,4 @@
-"""The register F-engine (8192- to 32768-point FFTs of real 2-bit samples) against the FP64
+"""The register F-engine (4096- to 32768-point FFTs of real 2-bit and complex 8-bit samples) against the FP64
 oracle where it can go wrong: every rotation order and both sidebands, one band per freq and
 sixteen bands, per-pol clock deltas and phase offsets (separate phasor tables), frames shorter
 than the stride of its sample loads, an FFT count that fills no workgroup, and slots with flagged
@@ -14,7 +14,7 @@ from fxcases import damaged_slot, record_errors, slot
 
 pytestmark = pytest.mark.gpu
 OFFS = (0, 1, 0)
-NCHAN = [4096, 8192, 16384]
+NCHAN = [2048, 4096, 8192, 16384]
 
 
 def _cfg(nchan, npol=2, nfreq=1, ffts=5, xe="fp32", **kw):
@@ -89,3 +89,11 @@ def test_damaged_slot(gpu, nchan, order, payload):
 @pytest.mark.parametrize("nchan", NCHAN)
 def test_short_frames(gpu, nchan):
     _check(lambda xe, m: _cfg(nchan, nfreq=8, xe=xe, payloadbytes=1024, fengine_mode=m))
+
+
+@pytest.mark.parametrize("nchan", [4096, 8192, 16384, 32768])
+@pytest.mark.parametrize("cplx,lsb,order,data_of", [(1, False, 1, slot), (1, True, 1, damaged_slot), (2, False, 1, damaged_slot),
+                                                    (1, True, 2, damaged_slot)])
+def test_complex(gpu, nchan, cplx, lsb, order, data_of):
+    _check(lambda xe, m: _cfg(nchan, xe=xe, nbits=8, complex_sampling=cplx, lsb=lsb, fringe_rot_order=order,
+                              fengine_mode=m), data_of=data_of)
