@@ -2148,8 +2148,8 @@ int run_subint(fxg_ctx* ctx, const int32_t offsets[3], const uint8_t* const* d_d
 
 // Autotuner: times one synthetic subint (zeroed slot buffers: the F-engine's control flow and
 // arithmetic do not depend on the data, only its loads of valid frames do) in every F-engine
-// launch form and workgroup size, and keeps the fastest.  The forms give bit-identical
-// results, so the choice only affects speed.
+// launch form and workgroup size, and keeps the fastest.  The forms give the same results up to
+// FP32 rounding (bit for bit where a thread holds the same butterfly positions).
 int autotune(fxg_ctx* ctx) {
   std::vector<std::pair<std::string, fxg_ctx::FChoice>> cand;
   auto add = [&](const char* name, int mode, int ntb, int mult) {

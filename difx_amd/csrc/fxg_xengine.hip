@@ -67,7 +67,9 @@ __global__ void __launch_bounds__(256) k_xmac_f32(XPlainArgs a) {
 // per row: a wave's reads, one row per lane, then hit distinct banks), double buffered, the next
 // stage's loads in flight while the current one is multiplied.  Rows past the group stay zero.
 // Runs of 64 FFTs are summed apart and then added to the total: one chain over 7800 FFTs of 10
-// stations was 1.3e-6 off the 64-bit result, runs of 256 1.1e-7.
+// stations was 1.3e-6 off the 64-bit result, runs of 256 1.1e-7.  Sums of up to 256 FFTs take runs
+// of 16: there the run's own rounding is what is left (63 FFTs of one baseline in one run were
+// 1.1e-7 off, the lane-per-channel sums in four parts before 9.3e-8).
 // R is the row count rounded up to 16, 32 or 64 (16x16x4 tiles, else 32x32x2).
 template <int R>
 struct XPTile {
@@ -82,7 +84,6 @@ struct XPTile {
   static constexpr int QN = TB * R * (CT / 2) / NTH;      // 16-byte loads per thread and stage
   static constexpr int NT = R == 64 ? 2 : 1;              // row tiles
   static constexpr int RR = R * R;                        // accumulators per channel
-  static constexpr int RUN = 64 / TB;                     // stages summed before they join the total
 };
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float float4_a8 __attribute__((ext_vector_type(4), aligned(8)));
@@ -98,6 +99,7 @@ __global__ void __launch_bounds__(XPTile<R>::NTH) k_xmac_f32_mat(XPMatArgs a) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int t0 = (int)((long long)it.split * a.nffts / g.nsplit);
   const int t1 = (int)((long long)(it.split + 1) * a.nffts / g.nsplit);
+  const int nrun = (t1 - t0 <= 256 ? 16 : 64) / TB;       // stages summed before they join the total
   const int nc = g.C - it.c0;                             // channels left (the last item may be short)
 
   for (int i = tid; i < 2 * T::STAGE; i += T::NTH) (&lds[0][0])[i] = make_float2(0.0f, 0.0f);
@@ -200,7 +202,7 @@ __global__ void __launch_bounds__(XPTile<R>::NTH) k_xmac_f32_mat(XPMatArgs a) {
   for (int t = t0; t < t1; t += TB, cur ^= 1) {
     load(t + TB);                                         // past the end: zeros, not used
     step(lds[cur]);
-    if (++run == T::RUN || t + TB >= t1) {
+    if (++run == nrun || t + TB >= t1) {
       run = 0;
 #pragma unroll
       for (int c = 0; c < CPW; ++c)
