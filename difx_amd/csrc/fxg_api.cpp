@@ -1593,9 +1593,15 @@ struct TimedLaunch {
   }
 };
 
+// Whether the matrix and register F-engines (and 1024 threads at 8192 points) run.  Not where the
+// spectral kurtosis reads 16-bit spectra: its values lie near zero, so the one in some thousand
+// 16-bit values that rounds the other way with them moves it by 3e-5 of its norm; those jobs keep
+// the rounding of the per-length kernels.
+bool fast_forms(const fxg_ctx* ctx) { return ctx->fsel.mat && !(ctx->kurt_on && ctx->xengine != FXG_X_FP32); }
+
 int ntb_for(const fxg_ctx* ctx, int L) {
   if (ctx->fsel.ntb) return ctx->fsel.ntb;
-  if (L == 8192 && ctx->fsel.mat) return 1024;   // no form asked for (see fe_minwaves)
+  if (L == 8192 && fast_forms(ctx)) return 1024;   // no form asked for (see fe_minwaves)
   return L >= 4096 ? 512 : 256;
 }
 
@@ -1828,7 +1834,7 @@ int build_items(fxg_ctx* ctx) {
 int launch_fengines(fxg_ctx* ctx, FengineArgs& fa, hipStream_t st) {
   const int nunits = fa.nffts_pad / 8;
   for (const auto& fc : ctx->fclasses) {
-    const bool reg = ctx->fsel.mat && fc.reg;
+    const bool reg = fast_forms(ctx) && fc.reg;
     if ((!fc.big && !reg) || ctx->fsel.mode == FXG_F_PERSISTENT) continue;
     fa.twiddle = ctx->d_twiddle + fc.tw_off;
     fa.dslist = ctx->d_dslist + fc.dsl_off;
@@ -1874,9 +1880,9 @@ int launch_fengines(fxg_ctx* ctx, FengineArgs& fa, hipStream_t st) {
     return FXG_OK;
   }
   for (const auto& fc : ctx->fclasses) {
-    if (fc.big || (ctx->fsel.mat && fc.reg)) continue;
+    if (fc.big || (fast_forms(ctx) && fc.reg)) continue;
     const int ncl = (int)fc.dsl.size();
-    if (ctx->fsel.mat && fc.mat) {
+    if (fast_forms(ctx) && fc.mat) {
       fa.dslist = ctx->d_dslist + fc.dsl_off;
       int nfr = 1;
       for (int d : fc.dsl) nfr = std::max(nfr, ctx->h_ds[d].nrecfreqs);

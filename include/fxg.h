@@ -148,7 +148,9 @@ typedef struct fxg_config {
 #define FXG_MAX_PHASECENTRES 16
 
 /* F-engine launch forms: one launch per FFT length (datastreams grouped by length), or every
- * length in one persistent launch whose workgroups take (length, datastream, part) work items. */
+ * length in one persistent launch whose workgroups take (length, datastream, part) work items.
+ * FXG_F_AUTO without fengine_threads: one launch per length, by the matrix kernel (2048 points of
+ * 2-bit samples) or the register kernel (4096 points and more) where they apply. */
 #define FXG_F_AUTO 0
 #define FXG_F_PER_LENGTH 1
 #define FXG_F_PERSISTENT 2

@@ -105,3 +105,17 @@ def test_damaged_slot(gpu, nchan, order):
 def test_short_frames(gpu, nchan):
     """16 bands of 1024-byte payloads: 256 samples per frame."""
     _check(lambda xe, m: _cfg(nchan, nfreq=8, xe=xe, payloadbytes=1024, fengine_mode=m))
+
+
+@pytest.mark.parametrize("nchan", [1024, 4096])
+def test_kurtosis_of_16bit_spectra_keeps_the_vector_kernels(gpu, nchan):
+    from difx_amd.core import FxCore
+    out = []
+    for mode in (0, 1):
+        cfg = _cfg(nchan, xe="fp16", fengine_mode=mode, fengine_threads=512 if mode and nchan == 4096 else 0)
+        data, ctrl = slot(cfg, OFFS, seed=44)
+        with FxCore(cfg) as core:
+            core.set_kurtosis(True)
+            core.processdata(OFFS, data, ctrl)
+            out.append(np.stack([core.getKurtosis(d, b, nchan) for d in range(2) for b in range(2)]))
+    np.testing.assert_array_equal(out[0], out[1])
