@@ -579,9 +579,11 @@ def copy_probe():
     print("copy probe: 1073741824 bytes copied", flush=True)
 
 
-# VALU lane instructions per input sample of k_fengine<2048,false,1,256> (real 2-bit, 16 bands
-# per word), from the SQ_INSTS_VALU counter summary committed with the kernel's profile.
-FENGINE_VALU_PER_SAMPLE_FILE = ROOT / "profiles" / "k_fengine_2048_valu_counters.txt"
+# VALU lane instructions per input sample of k_fmat<1> (real 2-bit, 16 bands per word), from the
+# SQ_INSTS_VALU counter summary committed with the kernel's profile, and its matrix operations
+# (96 v_mfma_f32_32x32x16_f16 per 4096 samples).
+FENGINE_VALU_PER_SAMPLE_FILE = ROOT / "profiles" / "k_fmat_counters.txt"
+FENGINE_MATRIX_FLOP_PER_SAMPLE = 96 * 2 * 32 * 32 * 16 / 4096
 VALU_PEAK_LANE_OPS = 256 * 64 * 2.4e9          # 256 CUs x 64 lanes x 2.4 GHz peak engine clock
 
 
@@ -662,7 +664,8 @@ def main():
         ach = vps * f_samples_per_launch / (f_avg_ms / 1e3)
         issue = {"bound": "valu", "achieved": ach, "peak": VALU_PEAK_LANE_OPS, "unit": "lane-instructions/s",
                  "frac": ach / VALU_PEAK_LANE_OPS, "valu_lane_instructions_per_sample": vps,
-                 "source": "profiles/k_fengine_2048_valu_counters.txt (SQ_INSTS_VALU x 64 / input samples)"}
+                 "matrix_tflops": FENGINE_MATRIX_FLOP_PER_SAMPLE * f_samples_per_launch / (f_avg_ms / 1e3) / 1e12,
+                 "source": "profiles/k_fmat_counters.txt (SQ_INSTS_VALU x 64 / input samples)"}
     plain = None
     if not args.no_plain:
         pcfg = workload_config("fp32")
@@ -713,7 +716,7 @@ def main():
         usamp = samples_per_subint(tcfg)
         forms = {}
         usteps = 5
-        for name, mode in (("per_length", 1), ("persistent", 2)):
+        for name, mode in (("per_length", 0), ("persistent", 2)):
             ucfg = uneven_config("fp16", fengine_mode=mode)
             print(f"[bench] uneven bands ({name} F-engine launch), 1 warmup + {usteps} steps", file=sys.stderr, flush=True)
             u = time_path(ucfg, usteps, 1, torch, dev, offsets)
@@ -807,10 +810,10 @@ def main():
                     "other_ms_per_step": hs["other_ms_per_step"],
                     "f_launches_per_step": nchunks_per_step,
                     "x_engine_useful_tflops": x_engine_flops(cfg, B) / (hs["x_ms_per_step"] / 1e3) / 1e12},
-        "roofline": {"kernel": "k_fengine<2048,false,1,256> (fused unpack+rotate+FFT+post-F, FP16 out)",
+        "roofline": {"kernel": "k_fmat<1> (fused unpack+rotate+FFT on the FP16 matrix cores+post-F, FP16 out)",
                      "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
                      "frac": achieved / HBM_PEAK_GBS,
-                     "traffic": measured_traffic(ROOT / "profiles" / "k_fengine_2048_traffic.txt", ffts_per_launch),
+                     "traffic": measured_traffic(ROOT / "profiles" / "k_fmat_traffic.txt", ffts_per_launch),
                      "avg_launch_ms": f_avg_ms, "algorithmic_bytes_per_launch": fbytes},
         "issue_roofline": issue,
         "plain_fp32": plain,
