@@ -457,24 +457,38 @@ __global__ void __launch_bounds__(256) k_xreduce_h(XReduceArgs a) {
   const int nch = min(XRH_CH, g.C - c0);
   const long long chf = (long long)ntp * 2048;
   const float* p = a.part + g.off + c0 * chf + (long long)tp * 2048 + i0 * 32;
+  // the places and the rows' scales are on their way while the parts are added: a small call's
+  // reduction is a chain of such loads (5.5 us with them in the loop below)
+  __shared__ float rs[8 + 32];
+  const long long* pairs = a.pairs + g.pair0;
+  constexpr int NE = 256 / (256 / XRH_CH);
+  long long pp[NE], pq[NE];
+#pragma unroll
+  for (int k = 0; k < NE; ++k) {
+    const int e = threadIdx.x / XRH_CH + k * (256 / XRH_CH), ri = ti * 32 + i0 + (e >> 5), rj = tj * 32 + (e & 31);
+    const bool in = ri < g.n && rj < g.n;
+    pp[k] = in ? pairs[ri * g.n + rj] : -1;
+    pq[k] = in && ti != tj ? pairs[rj * g.n + ri] : -1;
+  }
+  if (threadIdx.x < 40) {
+    const int r = threadIdx.x < 8 ? ti * 32 + i0 + (int)threadIdx.x : tj * 32 + (int)threadIdx.x - 8;
+    rs[threadIdx.x] = r < g.n ? a.xscale[g.scale_off + r] : 1.0f;
+  }
   xr_gather<2, XRH_CH>(s, p, p + 1024, chf, nch, 256, XRH_CS, g.nsplit, g.split_stride);
   __syncthreads();
   const int ch = threadIdx.x % XRH_CH;
   if (ch >= nch) return;
-  const long long* pairs = a.pairs + g.pair0;
   const float* sc = s + ch * XRH_CS;
-#pragma unroll 4
-  for (int e = threadIdx.x / XRH_CH; e < 256; e += 256 / XRH_CH) {
-    const int i = e >> 5, j = e & 31, ri = ti * 32 + i0 + i, rj = tj * 32 + j;
-    if (ri >= g.n || rj >= g.n) continue;
-    const long long p = pairs[ri * g.n + rj], q = ti == tj ? -1 : pairs[rj * g.n + ri];
-    if (p == -1 && q == -1) continue;
-    const float inv = 1.0f / (a.xscale[g.scale_off + ri] * a.xscale[g.scale_off + rj]);
+#pragma unroll
+  for (int n = 0; n < NE; ++n) {
+    if (pp[n] == -1 && pq[n] == -1) continue;
+    const int e = threadIdx.x / XRH_CH + n * (256 / XRH_CH), i = e >> 5, j = e & 31;
+    const float inv = 1.0f / (rs[i] * rs[8 + j]);
     const int k = mfma_idx(i, j);
     float2 v = make_float2(sc[k] * inv, sc[256 + k] * inv);
-    if (ri == rj) v.y = 0.0f;                              // x conj(x) is real
-    xr_put(a, p, c0 + ch, v);
-    xr_put(a, q, c0 + ch, make_float2(v.x, -v.y));
+    if (ti == tj && i0 + i == j) v.y = 0.0f;               // x conj(x) is real
+    xr_put(a, pp[n], c0 + ch, v);
+    xr_put(a, pq[n], c0 + ch, make_float2(v.x, -v.y));
   }
 }
 
