@@ -1053,9 +1053,11 @@ int tile_width_log(const DevXGroup& g, int want) {
 }
 
 // Splits of the X-engine's FFT loop: enough workgroups for the device where the channel tiles
-// alone (`units` workgroups) are too few, at least 16 FFTs each.
-int x_splits(const fxg_ctx* ctx, long long units, long long wanted) {
-  const long long most = std::max(1LL, (long long)std::min(ctx->chunkcap, ctx->B) / 16);
+// alone (`units` workgroups) are too few, at least `least` FFTs each: 16 on the FP32 matrix
+// instructions; 64 on the 16-bit ones, whose stages are longer (98 FFTs of 5 stations in six parts
+// took 52.5 us a call, in one 50.5 us; 500 FFTs of 6 stations in 31 84.6 us, in 7 65.4 us).
+int x_splits(const fxg_ctx* ctx, long long units, long long wanted, int least) {
+  const long long most = std::max(1LL, (long long)std::min(ctx->chunkcap, ctx->B) / least);
   return (int)std::max(1LL, std::min(most, wanted / std::max(1LL, units)));
 }
 
@@ -1147,7 +1149,7 @@ long long build_xplain(fxg_ctx* ctx) {
     long long units = 0;
     for (const auto& G : ctx->xp_groups) if (xp_class(G.nrows) == R) units += (G.C + ct - 1) / ct;
     if (!units) continue;
-    const int ns = x_splits(ctx, units, 4LL * ctx->ncu);
+    const int ns = x_splits(ctx, units, 4LL * ctx->ncu, 16);
     const int item0 = (int)ctx->xp_items.size();
     for (size_t gi = 0; gi < ctx->xp_groups.size(); ++gi) {
       XPGroup& G = ctx->xp_groups[gi];
@@ -1274,7 +1276,7 @@ int build_engines(fxg_ctx* ctx, int chunk_req) {
       const DevXGroup& G = ctx->groups[g0];
       for (g1 = g0; g1 < ctx->groups.size() && ctx->groups[g1].ntile == G.ntile && ctx->groups[g1].C == G.C; ++g1) {}
       const long long units = (long long)(g1 - g0) * (G.C >> G.twlog);
-      const int ns = x_splits(ctx, units, 2LL * ctx->ncu);
+      const int ns = x_splits(ctx, units, 2LL * ctx->ncu, 64);
       for (size_t g = g0; g < g1; ++g) ctx->groups[g].nsplit = ns;
     }
     long long off = 0, aoff = 0, soff = 0;
