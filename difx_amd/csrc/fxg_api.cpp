@@ -1364,12 +1364,23 @@ int build_engines(fxg_ctx* ctx, int chunk_req) {
     for (int d = 0; d < nds; ++d) {
       const fxg_datastream& s = ctx->dss[d];
       const int C = ctx->h_ds[d].C;
-      std::vector<long long> aacc(s.nrecbands), xacc(s.nrecbands, -1);
-      for (int b = 0; b < s.nrecbands; ++b) aacc[b] = add_prod(d, b, 0, d, b, 0, C);
-      if (ctx->crossautos)
+      // only bands that the results hold, themselves or through a zoom window: a product that
+      // nothing reads would still be stored
+      std::vector<char> wanted(s.nrecbands, 0);
+      for (int b = 0; b < s.nrecbands + s.nzoombands; ++b) {
+        const int fi = freq_of_band(s, b);
+        if (!(ctx->used[fi] || ctx->equiv[fi])) continue;
+        int rec, choff;
+        band_source(s, b, &rec, &choff);
+        wanted[rec] = 1;
+      }
+      std::vector<long long> aacc(s.nrecbands, -1), xacc(s.nrecbands, -1);
+      for (int b = 0; b < s.nrecbands; ++b)
+        if (wanted[b]) aacc[b] = add_prod(d, b, 0, d, b, 0, C);
+      if (ctx->crossautos && bpa == 2)
         for (int b = 0; b < s.nrecbands; ++b) {
           int pb = crosspol_partner(s, b);
-          if (pb >= 0) xacc[b] = add_prod(d, b, 0, d, pb, 0, C);
+          if (wanted[b] && pb >= 0) xacc[b] = add_prod(d, b, 0, d, pb, 0, C);
         }
       const int cavg = ctx->freqs[s.recfreq_index[0]].chanavg;
       long long idx = ctx->acoff[d];
@@ -1398,7 +1409,6 @@ int build_engines(fxg_ctx* ctx, int chunk_req) {
         }
       }
     }
-    ctx->xacc_len = acc;
     const long long plen = build_xplain(ctx);
     if (!ctx->xp_items.empty()) {
       if (int rc = dev_malloc(ctx, (void**)&ctx->d_vacc, (long long)sizeof(float) * plen)) return rc;
@@ -1489,7 +1499,6 @@ int build_engines(fxg_ctx* ctx, int chunk_req) {
         }
       }
     }
-    ctx->xacc_len = acc;
   }
   // products that go to the results channel by channel (one phase centre, no averaging, no other
   // reader such as a zoom window) are written there by the reduction itself
@@ -1520,7 +1529,12 @@ int build_engines(fxg_ctx* ctx, int chunk_req) {
     ctx->xr_maxC = std::max(ctx->xr_maxC, X.C);
     ctx->xr_maxtp = std::max(ctx->xr_maxtp, X.ntile * (X.ntile + 1) / 2);
   }
-  if (ctx->finp.empty()) ctx->xacc_len = 0;        // nothing reads a product accumulator
+  // the accumulators reach as far as the products stored there
+  ctx->xacc_len = 0;
+  for (const auto& X : ctx->xr_groups)
+    for (int k = 0; k < X.n * X.n; ++k)
+      if (ctx->xr_pairs[X.pair0 + k] >= 0) ctx->xacc_len = std::max(ctx->xacc_len, ctx->xr_pairs[X.pair0 + k] + X.C);
+  for (const auto& p : ctx->prods_rest) ctx->xacc_len = std::max(ctx->xacc_len, p.acc_off + p.nchan);
   if (int rc = dev_malloc(ctx, (void**)&ctx->d_xacc, (long long)sizeof(float2) * std::max<long long>(ctx->xacc_len, 2))) return rc;
   if (int rc = dev_upload(ctx, &ctx->d_finp, ctx->finp)) return rc;
   if (int rc = dev_upload(ctx, &ctx->d_xr_groups, ctx->xr_groups)) return rc;
@@ -3333,6 +3347,40 @@ int fxg_autotune_report(const fxg_ctx* ctx, char* buf, int32_t len) {
   }
   std::strncpy(buf, r.c_str(), (size_t)len - 1);
   buf[len - 1] = 0;
+  return FXG_OK;
+}
+
+// The extents of the X-engine's stores, for tests of the tables of any context (a host-only one
+// included): out = {entries of the product accumulators, end of the furthest store into them,
+// entries of the results, end of the furthest store into them, end of the furthest read of the
+// product accumulators, reads of entries that nothing stores}.  Entries are complex values.
+int fxg_x_extents(const fxg_ctx* ctx, int64_t out[6]) {
+  if (!ctx || !out) return FXG_E_INVALID;
+  std::vector<std::pair<long long, long long>> st;      // stores into the product accumulators
+  long long aend = 0, rend = 0, read = 0, lost = 0;
+  for (const auto& X : ctx->xr_groups)
+    for (int k = 0; k < X.n * X.n; ++k) {
+      const long long p = ctx->xr_pairs[X.pair0 + k];
+      if (p >= 0) st.push_back({p, p + X.C});
+      else if (p < -1) rend = std::max(rend, -2 - p + X.C);
+    }
+  for (const auto& p : ctx->prods_rest) st.push_back({p.acc_off, p.acc_off + p.nchan});
+  std::sort(st.begin(), st.end());
+  for (const auto& s : st) aend = std::max(aend, s.second);
+  for (const auto& e : ctx->finp) {
+    const int np = ctx->nphase > 1 && e.bl >= 0 ? ctx->nphase : 1;
+    rend = std::max(rend, (long long)e.dst + (long long)(np - 1) * e.pcstride + e.nout);
+    const long long r1 = e.src + (long long)e.nout * e.avg;
+    read = std::max(read, r1);
+    auto it = std::upper_bound(st.begin(), st.end(), std::pair<long long, long long>(e.src, 1LL << 62));
+    if (it == st.begin() || r1 > (--it)->second) ++lost;
+  }
+  out[0] = std::max<long long>(ctx->xacc_len, 2);
+  out[1] = aend;
+  out[2] = ctx->coreresultlength;
+  out[3] = rend;
+  out[4] = read;
+  out[5] = lost;
   return FXG_OK;
 }
 

@@ -1,0 +1,79 @@
+"""Where the X-engines store their sums, walked on the host: every store into the product
+accumulators and the results, and every read of the accumulators, lies inside its buffer, and
+every read finds a stored product.  The tables are those of a host-only context, the same as a
+device context's.  The configurations are the ones whose recorded bands are not all products:
+parallel hands only, a recorded freq that no baseline correlates, zoom windows with and without
+their parents, channel averaging, several phase centres, and rows beyond the matrix tiles."""
+import ctypes as C
+
+import pytest
+
+from difx_amd import config as cf
+from difx_amd.core import load_library
+from fxcases import case_cfg3, case_offsets, case_usb_lsb, with_phase_centres
+
+
+def parallel_hands(xe, stations=4, nchan=1024, **kw):
+    cfg = cf.standard_config(stations, 2, [4800.0], 32.0, nchan, subint_ns=16 * nchan * 1000 // 32, xengine=xe, seed=51,
+                             max_delay_us=50.0, **kw)
+    for b in cfg.baselines:
+        b.freqs = [(fi, prods[:2]) for fi, prods in b.freqs]
+    return cfg
+
+
+def uncorrelated_freq(xe, npol=1, nchan=1024, **kw):
+    """Two recorded freqs, of which the baselines correlate the first."""
+    cfg = cf.standard_config(4, npol, [4800.0, 4840.0], 32.0, nchan, subint_ns=16 * nchan * 1000 // 32, xengine=xe,
+                             seed=52, max_delay_us=50.0, **kw)
+    for b in cfg.baselines:
+        b.freqs = b.freqs[:1]
+    return cfg
+
+
+def zooms_alone(xe):
+    return cf.batched_config(3, [(32.0, 128, [4800.0, 4832.0])], [(0, 0, 2.0, 4.0), (0, 1, 28.0, 4.0)],
+                             subint_ns=16 * 4000, npol=2, xengine=xe, seed=53, max_delay_us=50.0, correlate_parents=False)
+
+
+def averaged(cfg, n=4):
+    for f in cfg.freqs:
+        f.chanavg = n
+    return cfg
+
+
+SHAPES = {
+    "parallel hands": parallel_hands,
+    "parallel hands, no cross autos": lambda xe: parallel_hands(xe, write_cross_autocorrs=False),
+    "parallel hands averaged": lambda xe: averaged(parallel_hands(xe)),
+    "uncorrelated freq": uncorrelated_freq,
+    "uncorrelated freq dual pol": lambda xe: uncorrelated_freq(xe, npol=2),
+    "uncorrelated freq averaged": lambda xe: averaged(uncorrelated_freq(xe)),
+    "zooms": lambda xe: case_cfg3(B=16, xengine=xe),
+    "zooms alone": zooms_alone,
+    "offsets, averaged": lambda xe: case_offsets(B=16, xengine=xe),
+    "usb x lsb": lambda xe: case_usb_lsb(B=16, xengine=xe),
+    "phase centres": lambda xe: with_phase_centres(parallel_hands(xe)),
+    "phase centres, uncorrelated freq": lambda xe: with_phase_centres(uncorrelated_freq(xe, npol=2)),
+    "one baseline of two freqs": lambda xe: uncorrelated_freq(xe, nchan=128),
+    "72 rows": lambda xe: cf.standard_config(36, 2, [4800.0], 32.0, 128, subint_ns=16 * 4000, xengine=xe, seed=54),
+}
+
+
+@pytest.mark.parametrize("xe", ["fp32", "fp16", "bf16"])
+@pytest.mark.parametrize("shape", sorted(SHAPES))
+def test_every_target_lies_inside_its_buffer(shape, xe):
+    if xe != "fp32" and shape == "72 rows":
+        pytest.skip("the 16-bit X-engine takes 64 rows")
+    lib = load_library()
+    fc, keep = SHAPES[shape](xe).to_abi()
+    h = C.c_void_p()
+    assert lib.fxg_create_layout(C.byref(fc), C.byref(h)) == 0, lib.fxg_last_error(None)
+    out = (C.c_int64 * 6)()
+    lib.fxg_x_extents.argtypes = [C.c_void_p, C.POINTER(C.c_int64)]
+    assert lib.fxg_x_extents(h, out) == 0
+    lib.fxg_destroy(h)
+    acc, acc_stored, res, res_stored, acc_read, lost = out
+    print(shape, xe, list(out))
+    assert acc_stored <= acc and acc_read <= acc, (acc_stored, acc_read, acc)
+    assert 0 < res_stored <= res
+    assert lost == 0
