@@ -1052,12 +1052,40 @@ int tile_width_log(const DevXGroup& g, int want) {
   return (want == 4 && g.ntile == 1 && g.C % 16 == 0) ? 4 : 3;
 }
 
+// The uv-shift intervals of a subint: each Core thread's range of FFTs, in steps of at most
+// getMaxNSBetweenXCAvg (a multiple of the buffered FFTs).
+void build_intervals(fxg_ctx* ctx) {
+  ctx->ivals.clear();
+  if (ctx->nphase <= 1) return;
+  const int B = ctx->B;
+  const double blockns = (double)ctx->subint_ns / (double)B;
+  int maxxc = (int)((double)ctx->maxns_xc / blockns);
+  maxxc -= maxxc % ctx->nbuffered;
+  if (maxxc == 0) maxxc = ctx->nbuffered;
+  int start = 0, nblk = 0;
+  for (int t = 0; t < ctx->nthreads; ++t) {
+    start += nblk;
+    nblk = B / ctx->nthreads + (t < B % ctx->nthreads ? 1 : 0);
+    for (int k = 0, sh = 0; k < nblk; k += maxxc, ++sh) {
+      const int n = std::min(maxxc, nblk - k);
+      ctx->ivals.push_back({start + k, n, (start + (double)sh * maxxc + n / 2.0) * blockns, n * blockns});
+    }
+  }
+}
+
 // Splits of the X-engine's FFT loop: enough workgroups for the device where the channel tiles
 // alone (`units` workgroups) are too few, at least `least` FFTs each: 16 on the FP32 matrix
 // instructions; 64 on the 16-bit ones, whose stages are longer (98 FFTs of 5 stations in six parts
-// took 52.5 us a call, in one 50.5 us; 500 FFTs of 6 stations in 31 84.6 us, in 7 65.4 us).
+// took 52.5 us a call, in one 50.5 us; 500 FFTs of 6 stations in 31 84.6 us, in 7 65.4 us).  The
+// loop runs over a chunk, or with several phase centres over one uv-shift interval of it.
+int x_longest(const fxg_ctx* ctx) {
+  int n = std::min(ctx->chunkcap, ctx->B), iv = 0;
+  for (const auto& i : ctx->ivals) iv = std::max(iv, i.n);
+  return ctx->ivals.empty() ? n : std::min(n, iv);
+}
+
 int x_splits(const fxg_ctx* ctx, long long units, long long wanted, int least) {
-  const long long most = std::max(1LL, (long long)std::min(ctx->chunkcap, ctx->B) / least);
+  const long long most = std::max(1LL, (long long)x_longest(ctx) / least);
   return (int)std::max(1LL, std::min(most, wanted / std::max(1LL, units)));
 }
 
@@ -1667,21 +1695,6 @@ int build_uvshift(fxg_ctx* ctx) {
     q.lsb = fr.lsb;
     q.rs = ctx->rs;
     q.nsteps = (fr.nchan / ctx->xms) * (ctx->xms / ctx->rs);
-  }
-  const int B = ctx->B;
-  const double blockns = (double)ctx->subint_ns / (double)B;
-  int maxxc = (int)((double)ctx->maxns_xc / blockns);
-  maxxc -= maxxc % ctx->nbuffered;
-  if (maxxc == 0) maxxc = ctx->nbuffered;
-  ctx->ivals.clear();
-  int start = 0, nblk = 0;
-  for (int t = 0; t < ctx->nthreads; ++t) {
-    start += nblk;
-    nblk = B / ctx->nthreads + (t < B % ctx->nthreads ? 1 : 0);
-    for (int k = 0, sh = 0; k < nblk; k += maxxc, ++sh) {
-      const int n = std::min(maxxc, nblk - k);
-      ctx->ivals.push_back({start + k, n, (start + (double)sh * maxxc + n / 2.0) * blockns, n * blockns});
-    }
   }
   const int nb = ctx->nbl;
   ctx->uvdec_idx.clear();
@@ -2620,6 +2633,7 @@ int create_impl(const fxg_config* cfg, fxg_ctx** out, bool dry) {
       rc = fail(ctx, FXG_E_HIP, "stream create");
   }
   if (rc == FXG_OK) rc = build_tables(ctx);
+  if (rc == FXG_OK) build_intervals(ctx);
   if (rc == FXG_OK) rc = build_engines(ctx, cfg->chunk_ffts);
   if (rc == FXG_OK) rc = build_items(ctx);
   if (rc == FXG_OK) rc = build_uvshift(ctx);
@@ -3353,8 +3367,9 @@ int fxg_autotune_report(const fxg_ctx* ctx, char* buf, int32_t len) {
 // The extents of the X-engine's stores, for tests of the tables of any context (a host-only one
 // included): out = {entries of the product accumulators, end of the furthest store into them,
 // entries of the results, end of the furthest store into them, end of the furthest read of the
-// product accumulators, reads of entries that nothing stores}.  Entries are complex values.
-int fxg_x_extents(const fxg_ctx* ctx, int64_t out[6]) {
+// product accumulators, reads of entries that nothing stores, FFTs of the longest run of an
+// X-engine loop, most parts that one is split into}.  Entries are complex values.
+int fxg_x_extents(const fxg_ctx* ctx, int64_t out[8]) {
   if (!ctx || !out) return FXG_E_INVALID;
   std::vector<std::pair<long long, long long>> st;      // stores into the product accumulators
   long long aend = 0, rend = 0, read = 0, lost = 0;
@@ -3381,6 +3396,9 @@ int fxg_x_extents(const fxg_ctx* ctx, int64_t out[6]) {
   out[3] = rend;
   out[4] = read;
   out[5] = lost;
+  out[6] = x_longest(ctx);
+  out[7] = 1;
+  for (const auto& X : ctx->xr_groups) out[7] = std::max<long long>(out[7], X.nsplit);
   return FXG_OK;
 }
 

@@ -59,21 +59,39 @@ SHAPES = {
 }
 
 
+def extents(cfg):
+    lib = load_library()
+    fc, keep = cfg.to_abi()
+    h = C.c_void_p()
+    assert lib.fxg_create_layout(C.byref(fc), C.byref(h)) == 0, lib.fxg_last_error(None)
+    out = (C.c_int64 * 8)()
+    lib.fxg_x_extents.argtypes = [C.c_void_p, C.POINTER(C.c_int64)]
+    assert lib.fxg_x_extents(h, out) == 0
+    lib.fxg_destroy(h)
+    return list(out)
+
+
 @pytest.mark.parametrize("xe", ["fp32", "fp16", "bf16"])
 @pytest.mark.parametrize("shape", sorted(SHAPES))
 def test_every_target_lies_inside_its_buffer(shape, xe):
     if xe != "fp32" and shape == "72 rows":
         pytest.skip("the 16-bit X-engine takes 64 rows")
-    lib = load_library()
-    fc, keep = SHAPES[shape](xe).to_abi()
-    h = C.c_void_p()
-    assert lib.fxg_create_layout(C.byref(fc), C.byref(h)) == 0, lib.fxg_last_error(None)
-    out = (C.c_int64 * 6)()
-    lib.fxg_x_extents.argtypes = [C.c_void_p, C.POINTER(C.c_int64)]
-    assert lib.fxg_x_extents(h, out) == 0
-    lib.fxg_destroy(h)
-    acc, acc_stored, res, res_stored, acc_read, lost = out
-    print(shape, xe, list(out))
+    acc, acc_stored, res, res_stored, acc_read, lost, _, _ = out = extents(SHAPES[shape](xe))
+    print(shape, xe, out)
     assert acc_stored <= acc and acc_read <= acc, (acc_stored, acc_read, acc)
     assert 0 < res_stored <= res
     assert lost == 0
+
+
+@pytest.mark.parametrize("xe,least", [("fp32", 16), ("fp16", 64), ("bf16", 64)])
+@pytest.mark.parametrize("ffts,interval,chunk,longest", [(1200, 0, 0, 1200), (1200, 0, 264, 264), (1200, 40, 0, 40),
+                                                        (1200, 100, 0, 100), (1200, 400, 264, 264)])
+def test_parts_of_a_run_keep_their_length(xe, least, ffts, interval, chunk, longest):
+    """No loop of the X-engine is split into parts shorter than its least, whatever bounds the loop:
+    the subint, a chunk of it, or a uv-shift interval with several phase centres."""
+    cfg = cf.standard_config(4, 2, [4800.0], 32.0, 128, subint_ns=ffts * 4000, xengine=xe, seed=58, chunk_ffts=chunk)
+    if interval:
+        with_phase_centres(cfg, P=2, interval_ffts=interval, threads=3)
+    *_, run, parts = extents(cfg)
+    assert run == longest
+    assert 1 <= parts <= max(1, longest // least)
