@@ -174,7 +174,7 @@ struct fxg_ctx {
   std::vector<XPGroup> xp_groups;
   std::vector<long long> xp_rows;
   std::vector<XPItem> xp_items;
-  struct XPClass { int R, item0, nitems; };
+  struct XPClass { int R, nsplit, item0, nitems; };
   std::vector<XPClass> xp_classes;
   std::vector<DevProd> prods_rest;
   XPGroup* d_xp_groups = nullptr;
@@ -1197,7 +1197,7 @@ long long build_xplain(fxg_ctx* ctx) {
           for (int h = 0; h < 16; h += ct)
             for (int c0 = c + h; c0 < std::min(G.C, c + 8 * 16); c0 += 16) ctx->xp_items.push_back(XPItem{(int)gi, c0, q});
     }
-    ctx->xp_classes.push_back({R, item0, (int)ctx->xp_items.size() - item0});
+    ctx->xp_classes.push_back({R, ns, item0, (int)ctx->xp_items.size() - item0});
   }
   return off;
 }
@@ -2121,7 +2121,7 @@ int run_subint(fxg_ctx* ctx, const int32_t offsets[3], const uint8_t* const* d_d
       ba.first = first;
       for (const auto& xc : ctx->xp_classes) {
         ba.items = ctx->d_xp_items + xc.item0;
-        if (fxg_launch_xplain_mat(ba, xc.R, xc.nitems, st)) return fail(ctx, FXG_E_HIP, "X-engine launch");
+        if (fxg_launch_xplain_mat(ba, xc.R, xc.nsplit, xc.nitems, st)) return fail(ctx, FXG_E_HIP, "X-engine launch");
       }
       if (!ctx->prods_rest.empty()) {
         XPlainArgs xa;

@@ -315,7 +315,7 @@ int fxg_launch_setup(const SetupArgs& a, int maxframes, hipStream_t st);
 int fxg_launch_unpack(const UnpackArgs& a, hipStream_t st);
 int fxg_launch_fengine(const FengineArgs& a, int L, int iscomplex, int nds, int ntb, hipStream_t st);
 int fxg_launch_fftparams(const FengineArgs& a, int nds, hipStream_t st);
-int fxg_launch_xplain_mat(const XPMatArgs& a, int R, int nitems, hipStream_t st);
+int fxg_launch_xplain_mat(const XPMatArgs& a, int R, int nsplit, int nitems, hipStream_t st);   // nsplit: of every group
 int fxg_launch_xreduce(const XReduceArgs& a, int mfma, int ngroups, int maxC, int maxtp, hipStream_t st);
 int fxg_launch_fpersist(const FengineArgs& a, const FItem* items, const IClass* cls, int ncls, int* counters,
                         int nwg, int ntb, int iscomplex, size_t lds, hipStream_t st);

@@ -68,8 +68,13 @@ __global__ void __launch_bounds__(256) k_xmac_f32(XPlainArgs a) {
 // stage's loads in flight while the current one is multiplied.  Rows past the group stay zero.
 // Runs of 64 FFTs are summed apart and then added to the total: one chain over 7800 FFTs of 10
 // stations was 1.3e-6 off the 64-bit result, runs of 256 1.1e-7.  Sums of up to 256 FFTs take runs
-// of 16: there the run's own rounding is what is left (63 FFTs of one baseline in one run were
-// 1.1e-7 off, the lane-per-channel sums in four parts before 9.3e-8).
+// of 8 and those of up to 64 runs of 4 (FINE: half a stage of the 16-row tiles, in a kernel of its
+// own, since in the long sums' the branch alone cost 1.4 %): there the run's own rounding is what is
+// left.  With the lane-per-channel sums in four parts, runs of 16 and these the results are off by
+// 9.6e-8, 1.09e-7 and 9.6e-8 for 24 FFTs of one baseline, by 1.10e-7, 9.4e-8 and 8.9e-8 for 200 of
+// 4 stations dual pol and by 1.41e-7, 1.41e-7 and 1.35e-7 for 63 of 20; 8 freqs of 1024 channels of
+// 10 stations and 63 FFTs take 143, now 146 us.  One matrix instruction at a time is worse again
+// (the total's own rounding) and spills at 64 rows.
 // R is the row count rounded up to 16, 32 or 64 (16x16x4 tiles, else 32x32x2).
 template <int R>
 struct XPTile {
@@ -88,7 +93,7 @@ struct XPTile {
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float float4_a8 __attribute__((ext_vector_type(4), aligned(8)));
 
-template <int R>
+template <int R, bool FINE>
 __global__ void __launch_bounds__(XPTile<R>::NTH) k_xmac_f32_mat(XPMatArgs a) {
   using T = XPTile<R>;
   constexpr int NT = T::NT, CPW = T::CPW, TB = T::TB, RS = T::RS, QN = T::QN;
@@ -99,7 +104,7 @@ __global__ void __launch_bounds__(XPTile<R>::NTH) k_xmac_f32_mat(XPMatArgs a) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int t0 = (int)((long long)it.split * a.nffts / g.nsplit);
   const int t1 = (int)((long long)(it.split + 1) * a.nffts / g.nsplit);
-  const int nrun = (t1 - t0 <= 256 ? 16 : 64) / TB;       // stages summed before they join the total
+  const int nrun = max(1, (t1 - t0 <= 64 ? 4 : t1 - t0 <= 256 ? 8 : 64) / TB);   // stages summed before they join the total
   const int nc = g.C - it.c0;                             // channels left (the last item may be short)
 
   for (int i = tid; i < 2 * T::STAGE; i += T::NTH) (&lds[0][0])[i] = make_float2(0.0f, 0.0f);
@@ -169,9 +174,23 @@ __global__ void __launch_bounds__(XPTile<R>::NTH) k_xmac_f32_mat(XPMatArgs a) {
   const bool im = R == 16 ? (lane >> 4) & 1 : lane >> 5;
   const int tk = R == 16 ? lane >> 5 : 0;
   const float sgn = im ? 1.0f : -1.0f;
+  auto fold = [&] {
+#pragma unroll
+    for (int c = 0; c < CPW; ++c)
+#pragma unroll
+      for (int ti = 0; ti < NT; ++ti)
+#pragma unroll
+        for (int tj = 0; tj < NT; ++tj)
+#pragma unroll
+          for (int r = 0; r < NREG; ++r) {
+            tot[c][ti][tj][r] += acc[c][ti][tj][r];
+            acc[c][ti][tj][r] = 0.0f;
+          }
+  };
   auto step = [&](const float2* s) {
 #pragma unroll
     for (int t = 0; t < TB; t += R == 16 ? 2 : 1) {
+      if (FINE && t == TB / 2) fold();
 #pragma unroll
       for (int c = 0; c < CPW; ++c) {
         float av[NT], bv[NT];
@@ -185,10 +204,9 @@ __global__ void __launch_bounds__(XPTile<R>::NTH) k_xmac_f32_mat(XPMatArgs a) {
         for (int ti = 0; ti < NT; ++ti)
 #pragma unroll
           for (int tj = 0; tj < NT; ++tj) {
-            if constexpr (R == 16)
-              acc[c][ti][tj] = __builtin_amdgcn_mfma_f32_16x16x4f32(av[ti], bv[tj], acc[c][ti][tj], 0, 0, 0);
-            else
-              acc[c][ti][tj] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[ti], bv[tj], acc[c][ti][tj], 0, 0, 0);
+            accv& v = acc[c][ti][tj];
+            if constexpr (R == 16) v = __builtin_amdgcn_mfma_f32_16x16x4f32(av[ti], bv[tj], v, 0, 0, 0);
+            else v = __builtin_amdgcn_mfma_f32_32x32x2f32(av[ti], bv[tj], v, 0, 0, 0);
           }
       }
     }
@@ -204,17 +222,7 @@ __global__ void __launch_bounds__(XPTile<R>::NTH) k_xmac_f32_mat(XPMatArgs a) {
     step(lds[cur]);
     if (++run == nrun || t + TB >= t1) {
       run = 0;
-#pragma unroll
-      for (int c = 0; c < CPW; ++c)
-#pragma unroll
-        for (int ti = 0; ti < NT; ++ti)
-#pragma unroll
-          for (int tj = 0; tj < NT; ++tj)
-#pragma unroll
-            for (int r = 0; r < NREG; ++r) {
-              tot[c][ti][tj][r] += acc[c][ti][tj][r];
-              acc[c][ti][tj][r] = 0.0f;
-            }
+      fold();
     }
     if (t + TB < t1) store(lds[cur ^ 1]);
     __syncthreads();
@@ -647,11 +655,13 @@ __global__ void k_fill(float* p, long long n, float v) {
 }
 
 // ---- host-side launchers -------------------------------------------------------------
-int fxg_launch_xplain_mat(const XPMatArgs& a, int R, int nitems, hipStream_t st) {
+int fxg_launch_xplain_mat(const XPMatArgs& a, int R, int nsplit, int nitems, hipStream_t st) {
   const dim3 grid(nitems);
-  if (R == 16) hipLaunchKernelGGL(k_xmac_f32_mat<16>, grid, dim3(XPTile<16>::NTH), 0, st, a);
-  else if (R == 32) hipLaunchKernelGGL(k_xmac_f32_mat<32>, grid, dim3(XPTile<32>::NTH), 0, st, a);
-  else hipLaunchKernelGGL(k_xmac_f32_mat<64>, grid, dim3(XPTile<64>::NTH), 0, st, a);
+  const bool fine = (a.nffts + nsplit - 1) / nsplit <= 64;
+  if (R == 16 && fine) hipLaunchKernelGGL((k_xmac_f32_mat<16, true>), grid, dim3(XPTile<16>::NTH), 0, st, a);
+  else if (R == 16) hipLaunchKernelGGL((k_xmac_f32_mat<16, false>), grid, dim3(XPTile<16>::NTH), 0, st, a);
+  else if (R == 32) hipLaunchKernelGGL((k_xmac_f32_mat<32, false>), grid, dim3(XPTile<32>::NTH), 0, st, a);
+  else hipLaunchKernelGGL((k_xmac_f32_mat<64, false>), grid, dim3(XPTile<64>::NTH), 0, st, a);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
