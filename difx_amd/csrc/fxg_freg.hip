@@ -287,6 +287,22 @@ __global__ void __launch_bounds__(L / 32 * RPlan<L>::G, 4) k_freg(FengineArgs ar
         const bool lsb = dsp->rf[f].lsb != 0;
         const uint32_t p0 = kb & 1 ? pk[1][0] : pk[0][0], p1 = kb & 1 ? pk[1][1] : pk[0][1];
         fence();
+        // order 2: the quadratic sub term^j, j = n/S (mode.cpp:1017-1024), of every eighth sample and
+        // its step from one sample to the next (a chain of 32 factors was 1.9 times as far off)
+        float2 qstart[4], qstep = make_float2(1.0f, 0.0f);
+        if (ORDER == 2) {
+          const int t = opaque(t0);
+          const float th = squad[t & (S - 1)];
+          float sn, cs;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            sincosf((float)(t / S + 8 * i * (NT / S)) * th, &sn, &cs);
+            qstart[i] = make_float2(cs, sn);
+          }
+          sincosf((float)(NT / S) * th, &sn, &cs);
+          qstep = make_float2(cs, sn);
+          fence();
+        }
         if (CPLX) {
           // complex 8-bit samples: both bytes in one load, sixteen in flight; an invalid sample
           // reads the buffer's first bytes, if it has any
@@ -319,15 +335,7 @@ __global__ void __launch_bounds__(L / 32 * RPlan<L>::G, 4) k_freg(FengineArgs ar
         {
           const int t = opaque(t0);
           const float2 sub = ORDER != 0 ? srot[t & (S - 1)] : make_float2(1.0f, 0.0f);
-          float2 qpow = make_float2(1.0f, 0.0f), qstep = make_float2(1.0f, 0.0f);
-          if (ORDER == 2) {                      // quadratic sub term^j, j = n/S (mode.cpp:1017-1024)
-            const float th = squad[t & (S - 1)];
-            float sn, cs;
-            sincosf((float)(t / S) * th, &sn, &cs);
-            qpow = make_float2(cs, sn);
-            sincosf((float)(NT / S) * th, &sn, &cs);
-            qstep = make_float2(cs, sn);
-          }
+          float2 qpow = make_float2(1.0f, 0.0f);
           const float2* __restrict__ step = srot + S + t / S;    // NT is a multiple of S
 #pragma unroll
           for (int s = 0; s < 32; ++s) {
@@ -336,6 +344,7 @@ __global__ void __launch_bounds__(L / 32 * RPlan<L>::G, 4) k_freg(FengineArgs ar
               v[s] = make_float2(x, 0.0f);
             } else {
               float2 rot = sub;
+              if (ORDER == 2 && s % 8 == 0) qpow = qstart[s / 8];
               if (ORDER == 2) { rot = cmul(sub, qpow); qpow = cmul(qpow, qstep); }
               rot = cmul(rot, step[s * (NT / S)]);
               v[s] = CPLX ? cmul(rot, v[s]) : make_float2(x * rot.x, x * rot.y);
