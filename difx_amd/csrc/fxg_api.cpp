@@ -196,6 +196,8 @@ struct fxg_ctx {
   XRGroup* d_xr_groups = nullptr;
   long long* d_xr_pairs = nullptr;
   int xr_maxC = 0, xr_maxtp = 0;
+  struct XRBatch { int g0, ng, f0, nf; };   // groups and the accumulation entries that read them
+  std::vector<XRBatch> xr_batches;
   float* d_xscale = nullptr;
   long long xscale_len = 0;
   // accumulation entries
@@ -1150,7 +1152,6 @@ long long build_xplain(fxg_ctx* ctx) {
     }
     XRGroup X;
     std::memset(&X, 0, sizeof(X));
-    X.kind = n <= 16 ? XR_S16 : XR_S32;
     X.n = n;
     X.C = G.C;
     X.ntile = n <= 32 ? 1 : 2;
@@ -1183,7 +1184,7 @@ long long build_xplain(fxg_ctx* ctx) {
       XPGroup& G = ctx->xp_groups[gi];
       if (xp_class(G.nrows) != R) continue;
       G.off = off;
-      G.split_stride = (long long)G.C * R * R;
+      G.split_stride = (long long)G.C * xp_floats(G.nrows);
       G.nsplit = ns;
       off += ns * G.split_stride;
       XRGroup& X = ctx->xr_groups[gi];
@@ -1200,6 +1201,60 @@ long long build_xplain(fxg_ctx* ctx) {
     ctx->xp_classes.push_back({R, ns, item0, (int)ctx->xp_items.size() - item0});
   }
   return off;
+}
+
+// Places the product accumulators that are left: those of the per-product kernel, which live through a
+// subint, and then the reduction's, which only pass from it to the accumulation.  The groups go through
+// the latter in batches of at most 64 MiB (or one group), so that jobs whose products are averaged or
+// have several phase centres need no second copy of all sums: 32 stations x 8 freqs x 8192 channels,
+// dual pol, 16-bit, averaged, 6820 -> 5896 MiB.
+void place_accumulators(fxg_ctx* ctx) {
+  constexpr long long BATCH = (64LL << 20) / (long long)sizeof(float2);
+  struct Slot { long long from, to; int n, batch; };
+  std::vector<Slot> slots;
+  long long rest = 0;
+  for (auto& p : ctx->prods_rest) {
+    slots.push_back({p.acc_off, rest, p.nchan, 0});
+    p.acc_off = rest;
+    rest += p.nchan;
+  }
+  ctx->xr_batches.clear();
+  ctx->xacc_len = rest;
+  const int ng = (int)ctx->xr_groups.size();
+  long long off = rest;
+  for (int g = 0; g < ng; ++g) {
+    const XRGroup& X = ctx->xr_groups[g];
+    long long* p = ctx->xr_pairs.data() + X.pair0;
+    long long len = 0;
+    for (int k = 0; k < X.n * X.n; ++k) len += p[k] >= 0 ? X.C : 0;
+    if (g == 0 || off - rest + len > BATCH) {
+      ctx->xr_batches.push_back({g, 0, 0, 0});
+      off = rest;
+    }
+    const int batch = (int)ctx->xr_batches.size() - 1;
+    ctx->xr_batches.back().ng++;
+    for (int k = 0; k < X.n * X.n; ++k)
+      if (p[k] >= 0) {
+        slots.push_back({p[k], off, X.C, batch});
+        p[k] = off;
+        off += X.C;
+      }
+    ctx->xacc_len = std::max(ctx->xacc_len, off);
+  }
+  if (ctx->xr_batches.empty()) ctx->xr_batches.push_back({0, 0, 0, 0});
+  std::sort(slots.begin(), slots.end(), [](const Slot& a, const Slot& b) { return a.from < b.from; });
+  std::vector<std::vector<FinProd>> fin(ctx->xr_batches.size());
+  for (FinProd e : ctx->finp) {                    // every entry reads a product that was made above
+    const Slot& s = *--std::upper_bound(slots.begin(), slots.end(), e.src, [](long long v, const Slot& t) { return v < t.from; });
+    e.src += s.to - s.from;
+    fin[s.batch].push_back(e);
+  }
+  ctx->finp.clear();
+  for (size_t k = 0; k < fin.size(); ++k) {
+    ctx->xr_batches[k].f0 = (int)ctx->finp.size();
+    ctx->xr_batches[k].nf = (int)fin[k].size();
+    ctx->finp.insert(ctx->finp.end(), fin[k].begin(), fin[k].end());
+  }
 }
 
 int build_engines(fxg_ctx* ctx, int chunk_req) {
@@ -1444,15 +1499,12 @@ int build_engines(fxg_ctx* ctx, int chunk_req) {
       if (int rc = dev_upload(ctx, &ctx->d_xp_rows, ctx->xp_rows)) return rc;
       if (int rc = dev_upload(ctx, &ctx->d_xp_items, ctx->xp_items)) return rc;
     }
-    if (!ctx->prods_rest.empty())
-      if (int rc = dev_upload(ctx, &ctx->d_prods_rest, ctx->prods_rest)) return rc;
   } else {
     // a pair table per group: the accumulator of each ordered row pair that a product uses
     for (size_t g = 0; g < ctx->groups.size(); ++g) {
       const DevXGroup& G = ctx->groups[g];
       XRGroup X;
       std::memset(&X, 0, sizeof(X));
-      X.kind = XR_H;
       X.n = G.nin;
       X.C = G.C;
       X.ntile = G.ntile;
@@ -1557,13 +1609,10 @@ int build_engines(fxg_ctx* ctx, int chunk_req) {
     ctx->xr_maxC = std::max(ctx->xr_maxC, X.C);
     ctx->xr_maxtp = std::max(ctx->xr_maxtp, X.ntile * (X.ntile + 1) / 2);
   }
-  // the accumulators reach as far as the products stored there
-  ctx->xacc_len = 0;
-  for (const auto& X : ctx->xr_groups)
-    for (int k = 0; k < X.n * X.n; ++k)
-      if (ctx->xr_pairs[X.pair0 + k] >= 0) ctx->xacc_len = std::max(ctx->xacc_len, ctx->xr_pairs[X.pair0 + k] + X.C);
-  for (const auto& p : ctx->prods_rest) ctx->xacc_len = std::max(ctx->xacc_len, p.acc_off + p.nchan);
+  place_accumulators(ctx);
   if (int rc = dev_malloc(ctx, (void**)&ctx->d_xacc, (long long)sizeof(float2) * std::max<long long>(ctx->xacc_len, 2))) return rc;
+  if (!ctx->prods_rest.empty())
+    if (int rc = dev_upload(ctx, &ctx->d_prods_rest, ctx->prods_rest)) return rc;
   if (int rc = dev_upload(ctx, &ctx->d_finp, ctx->finp)) return rc;
   if (int rc = dev_upload(ctx, &ctx->d_xr_groups, ctx->xr_groups)) return rc;
   if (int rc = dev_upload(ctx, &ctx->d_xr_pairs, ctx->xr_pairs)) return rc;
@@ -2056,15 +2105,17 @@ int run_subint(fxg_ctx* ctx, const int32_t offsets[3], const uint8_t* const* d_d
   auto accumulate = [&](const UvArgs& u) -> int {
     TimedLaunch tl(ctx, 2, st);
     XReduceArgs ra;
-    ra.groups = ctx->d_xr_groups;
     ra.pairs = ctx->d_xr_pairs;
     ra.part = ctx->d_vacc;
     ra.xscale = ctx->d_xscale;
     ra.acc = ctx->d_xacc;
     ra.res = d_results;
-    if (fxg_launch_xreduce(ra, mfma, (int)ctx->xr_groups.size(), ctx->xr_maxC, ctx->xr_maxtp, st) ||
-        fxg_launch_fin(ctx->d_finp, (int)ctx->finp.size(), ctx->maxoutp, ctx->d_xacc, d_results, u, st))
-      return fail(ctx, FXG_E_HIP, "accumulate launch");
+    for (const auto& b : ctx->xr_batches) {
+      ra.groups = ctx->d_xr_groups + b.g0;
+      if (fxg_launch_xreduce(ra, mfma, b.ng, ctx->xr_maxC, ctx->xr_maxtp, st) ||
+          fxg_launch_fin(ctx->d_finp + b.f0, b.nf, ctx->maxoutp, ctx->d_xacc, d_results, u, st))
+        return fail(ctx, FXG_E_HIP, "accumulate launch");
+    }
     return FXG_OK;
   };
   int first = 1;                                   // the accumulators start here
@@ -3368,27 +3419,36 @@ int fxg_autotune_report(const fxg_ctx* ctx, char* buf, int32_t len) {
 // included): out = {entries of the product accumulators, end of the furthest store into them,
 // entries of the results, end of the furthest store into them, end of the furthest read of the
 // product accumulators, reads of entries that nothing stores, FFTs of the longest run of an
-// X-engine loop, most parts that one is split into}.  Entries are complex values.
-int fxg_x_extents(const fxg_ctx* ctx, int64_t out[8]) {
+// X-engine loop, most parts that one is split into, batches of the accumulation}.  Entries are
+// complex values.
+int fxg_x_extents(const fxg_ctx* ctx, int64_t out[9]) {
   if (!ctx || !out) return FXG_E_INVALID;
-  std::vector<std::pair<long long, long long>> st;      // stores into the product accumulators
   long long aend = 0, rend = 0, read = 0, lost = 0;
-  for (const auto& X : ctx->xr_groups)
-    for (int k = 0; k < X.n * X.n; ++k) {
-      const long long p = ctx->xr_pairs[X.pair0 + k];
-      if (p >= 0) st.push_back({p, p + X.C});
-      else if (p < -1) rend = std::max(rend, -2 - p + X.C);
+  for (const auto& b : ctx->xr_batches) {
+    std::vector<std::pair<long long, long long>> st;    // stores into the product accumulators
+    for (int g = b.g0; g < b.g0 + b.ng; ++g) {
+      const XRGroup& X = ctx->xr_groups[g];
+      for (int k = 0; k < X.n * X.n; ++k) {
+        const long long p = ctx->xr_pairs[X.pair0 + k];
+        if (p >= 0) st.push_back({p, p + X.C});
+        else if (p < -1) rend = std::max(rend, -2 - p + X.C);
+      }
     }
-  for (const auto& p : ctx->prods_rest) st.push_back({p.acc_off, p.acc_off + p.nchan});
-  std::sort(st.begin(), st.end());
-  for (const auto& s : st) aend = std::max(aend, s.second);
-  for (const auto& e : ctx->finp) {
-    const int np = ctx->nphase > 1 && e.bl >= 0 ? ctx->nphase : 1;
-    rend = std::max(rend, (long long)e.dst + (long long)(np - 1) * e.pcstride + e.nout);
-    const long long r1 = e.src + (long long)e.nout * e.avg;
-    read = std::max(read, r1);
-    auto it = std::upper_bound(st.begin(), st.end(), std::pair<long long, long long>(e.src, 1LL << 62));
-    if (it == st.begin() || r1 > (--it)->second) ++lost;
+    for (const auto& p : ctx->prods_rest) st.push_back({p.acc_off, p.acc_off + p.nchan});
+    std::sort(st.begin(), st.end());
+    for (size_t k = 0; k < st.size(); ++k) {
+      aend = std::max(aend, st[k].second);
+      if (k && st[k].first < st[k - 1].second) ++lost;  // two stores into one entry
+    }
+    for (int f = b.f0; f < b.f0 + b.nf; ++f) {
+      const FinProd& e = ctx->finp[f];
+      const int np = ctx->nphase > 1 && e.bl >= 0 ? ctx->nphase : 1;
+      rend = std::max(rend, (long long)e.dst + (long long)(np - 1) * e.pcstride + e.nout);
+      const long long r1 = e.src + (long long)e.nout * e.avg;
+      read = std::max(read, r1);
+      auto it = std::upper_bound(st.begin(), st.end(), std::pair<long long, long long>(e.src, 1LL << 62));
+      if (it == st.begin() || r1 > (--it)->second) ++lost;
+    }
   }
   out[0] = std::max<long long>(ctx->xacc_len, 2);
   out[1] = aend;
@@ -3399,6 +3459,7 @@ int fxg_x_extents(const fxg_ctx* ctx, int64_t out[8]) {
   out[6] = x_longest(ctx);
   out[7] = 1;
   for (const auto& X : ctx->xr_groups) out[7] = std::max<long long>(out[7], X.nsplit);
+  out[8] = (int64_t)ctx->xr_batches.size();
   return FXG_OK;
 }
 

@@ -222,10 +222,18 @@ struct XPlainArgs {
 #define XP_MAXROWS 64       // rows per group (larger groups: per-product kernel)
 constexpr int xp_class(int nrows) { return nrows <= 16 ? 16 : nrows <= 32 ? 32 : 64; }
 constexpr int xp_ct(int R) { return R == 64 ? 8 : 16; }
+// A channel's accumulators: the n x n matrix S as tiles of up to 32 rows (and columns), the rows of a
+// tile one after the other, a tile padded to whole 16-byte words.  Rows past the group are left out: as
+// whole tiles 33 stations x 8 freqs x 16384 channels took 2.1 GiB, three times their products.
+__host__ __device__ constexpr int xp_rows(int n, int t) { return n - 32 * t < 32 ? n - 32 * t : 32; }
+__host__ __device__ constexpr int xp_tile(int n, int ti, int tj) {
+  return n <= 32 ? 0 : ti == 0 ? tj * 1024 : 32 * n + tj * 32 * (n - 32);
+}
+__host__ __device__ constexpr int xp_floats(int n) { return (n * n + 3) & ~3; }
 struct XPGroup {
   int nrows, C, row0;       // rows[row0 + i]: cf32 offset of (band, FFT 0, window start)
   int stride;               // cf32 entries between consecutive FFTs, the same for every row
-  long long off;            // float offset of its accumulators: per channel the R x R matrix S
+  long long off;            // float offset of its accumulators: per channel xp_floats(nrows)
   long long split_stride;   // floats between the accumulators of its splits
   int nsplit, pad;
 };
@@ -245,15 +253,13 @@ struct XPMatArgs {
 // Raw accumulator tiles of either X-engine into per-product rows of channels: the splits over
 // FFTs are summed in order and product (i, j) of a group goes, by its pair table entry p, to
 // acc[p + c] (p >= 0), straight to the results, res[-2 - p + c] (p <= -2), or nowhere (-1).
-#define XR_S16 0            // FP32, one 16 x 16 tile S per channel
-#define XR_S32 1            // FP32, ntile^2 32 x 32 tiles S per channel
-#define XR_H 2              // 16-bit, (re, im) 32 x 32 tiles of the lower tile pairs per channel
+// FP32: the matrix S per channel (xp_floats); 16-bit: (re, im) 32 x 32 tiles of the lower tile pairs.
 struct XRGroup {
-  int kind, n, C, ntile;
+  int n, C, ntile, pad;
   long long off;            // float offset of split 0, channel 0
   long long split_stride;
-  long long scale_off;      // XR_H: float offset of its per-row scales
-  int pair0;                // first entry of its n x n pair table 
+  long long scale_off;      // 16-bit: float offset of its per-row scales
+  int pair0;                // first entry of its n x n pair table
   int nsplit;
 };
 struct XReduceArgs {

@@ -88,7 +88,6 @@ struct XPTile {
   static constexpr int STAGE = TB * R * RS;
   static constexpr int QN = TB * R * (CT / 2) / NTH;      // 16-byte loads per thread and stage
   static constexpr int NT = R == 64 ? 2 : 1;              // row tiles
-  static constexpr int RR = R * R;                        // accumulators per channel
 };
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef float float4_a8 __attribute__((ext_vector_type(4), aligned(8)));
@@ -151,7 +150,8 @@ __global__ void __launch_bounds__(XPTile<R>::NTH) k_xmac_f32_mat(XPMatArgs a) {
   // accumulators, [channel of the wave][row tile][column tile][register]
   typedef float accv __attribute__((ext_vector_type(NREG)));
   accv acc[CPW][NT][NT];
-  float* part = a.part + g.off + it.split * g.split_stride + (long long)(it.c0 + wave * CPW) * T::RR + lane;
+  const int cs = xp_floats(g.nrows);                      // floats per channel
+  float* part = a.part + g.off + it.split * g.split_stride + (long long)(it.c0 + wave * CPW) * cs;
 #pragma unroll
   for (int c = 0; c < CPW; ++c)
 #pragma unroll
@@ -227,19 +227,25 @@ __global__ void __launch_bounds__(XPTile<R>::NTH) k_xmac_f32_mat(XPMatArgs a) {
     if (t + TB < t1) store(lds[cur ^ 1]);
     __syncthreads();
   }
+  // the group's rows only, tile by tile in row order
 #pragma unroll
-  for (int c = 0; c < CPW; ++c) {
-    if (wave * CPW + c >= nc) continue;
+  for (int ti = 0; ti < NT; ++ti)
 #pragma unroll
-    for (int ti = 0; ti < NT; ++ti)
+    for (int tj = 0; tj < NT; ++tj) {
+      const int h = xp_rows(g.nrows, ti), w = xp_rows(g.nrows, tj);
+      float* pt = part + xp_tile(g.nrows, ti, tj);
 #pragma unroll
-      for (int tj = 0; tj < NT; ++tj)
+      for (int r = 0; r < NREG; ++r) {
+        const int i = R == 16 ? 4 * (lane >> 4) + r : 8 * (r >> 2) + 4 * (lane >> 5) + (r & 3);
+        if (i >= h || row >= w) continue;
 #pragma unroll
-        for (int r = 0; r < NREG; ++r) {
-          float* p = part + c * T::RR + (ti * NT + tj) * 1024 + r * 64;
+        for (int c = 0; c < CPW; ++c) {
+          if (wave * CPW + c >= nc) continue;
+          float* p = pt + c * cs + i * w + row;
           *p = a.first ? tot[c][ti][tj][r] : *p + tot[c][ti][tj][r];
         }
-  }
+      }
+    }
 }
 
 template <typename V8>
@@ -417,8 +423,6 @@ __device__ __forceinline__ int mfma_idx(int i, int j) {
   const int l = ((i >> 2) & 1) * 32 + j;
   return r * 64 + l;
 }
-// The same for a 16x16 accumulator: register r of lane l holds (4 (l / 16) + r, l % 16).
-__device__ __forceinline__ int mfma_idx16(int i, int j) { return (i & 3) * 64 + (i >> 2) * 16 + j; }
 
 // The raw accumulator tiles to the products: a workgroup reads a block of tiles of a few
 // channels of one group into LDS, whole lines at a time, summing the splits in order, and then
@@ -509,31 +513,28 @@ __global__ void __launch_bounds__(256) k_xreduce_s(XReduceArgs a) {
   int ti = 0, tj = blockIdx.z;
   while (tj > ti) { ++ti; tj -= ti; }
   if (c0 >= g.C || ti >= g.ntile) return;
-  const bool s16 = g.kind == XR_S16;
-  const int tile = s16 ? 256 : 1024;
+  const int h = xp_rows(g.n, ti), w = xp_rows(g.n, tj), len = (h * w + 3) & ~3;
   const int nch = min(XRS_CH, g.C - c0);
-  const long long chf = (long long)g.ntile * g.ntile * tile;
+  const long long chf = xp_floats(g.n);
   const float* p = a.part + g.off + c0 * chf;
   if (ti == tj)
-    xr_gather<1, XRS_CH>(s, p + (long long)(ti * g.ntile + tj) * tile, nullptr, chf, nch, tile, XRS_CS, g.nsplit, g.split_stride);
+    xr_gather<1, XRS_CH>(s, p + xp_tile(g.n, ti, tj), nullptr, chf, nch, len, XRS_CS, g.nsplit, g.split_stride);
   else
-    xr_gather<2, XRS_CH>(s, p + (long long)(ti * g.ntile + tj) * tile, p + (long long)(tj * g.ntile + ti) * tile, chf, nch,
-                         tile, XRS_CS, g.nsplit, g.split_stride);
+    xr_gather<2, XRS_CH>(s, p + xp_tile(g.n, ti, tj), p + xp_tile(g.n, tj, ti), chf, nch, len, XRS_CS, g.nsplit, g.split_stride);
   __syncthreads();
-  const int w = s16 ? 16 : 32, wl = s16 ? 4 : 5;
   const int ch = threadIdx.x % XRS_CH;
   if (ch >= nch) return;
   const long long* pairs = a.pairs + g.pair0;
   const float* sc = s + ch * XRS_CS;
-  const float* st = sc + (ti == tj ? 0 : tile);
+  const float* st = sc + (ti == tj ? 0 : len);
+  const int wl = w <= 16 ? 4 : 5;
 #pragma unroll 4
-  for (int e = threadIdx.x / XRS_CH; e < w * w; e += 256 / XRS_CH) {
-    const int i = e >> wl, j = e & (w - 1), ri = ti * 32 + i, rj = tj * 32 + j;
-    if (ri >= g.n || rj >= g.n) continue;
+  for (int e = threadIdx.x / XRS_CH; e < h << wl; e += 256 / XRS_CH) {
+    const int i = e >> wl, j = e & ((1 << wl) - 1), ri = ti * 32 + i, rj = tj * 32 + j;
+    if (j >= w) continue;
     const long long p = pairs[ri * g.n + rj], q = ti == tj ? -1 : pairs[rj * g.n + ri];
     if (p == -1 && q == -1) continue;
-    const float x = sc[s16 ? mfma_idx16(i, j) : mfma_idx(i, j)];
-    const float y = st[s16 ? mfma_idx16(j, i) : mfma_idx(j, i)];
+    const float x = sc[i * w + j], y = st[j * h + i];
     const float2 v = make_float2(0.5f * (x + y), 0.5f * (x - y));   // i = j: imaginary part 0
     xr_put(a, p, c0 + ch, v);
     xr_put(a, q, c0 + ch, make_float2(v.x, -v.y));

@@ -9,7 +9,7 @@ import ctypes as C
 import pytest
 
 from difx_amd import config as cf
-from difx_amd.core import load_library
+from difx_amd.core import footprint, load_library
 from fxcases import case_cfg3, case_offsets, case_usb_lsb, with_phase_centres
 
 
@@ -64,7 +64,7 @@ def extents(cfg):
     fc, keep = cfg.to_abi()
     h = C.c_void_p()
     assert lib.fxg_create_layout(C.byref(fc), C.byref(h)) == 0, lib.fxg_last_error(None)
-    out = (C.c_int64 * 8)()
+    out = (C.c_int64 * 9)()
     lib.fxg_x_extents.argtypes = [C.c_void_p, C.POINTER(C.c_int64)]
     assert lib.fxg_x_extents(h, out) == 0
     lib.fxg_destroy(h)
@@ -76,7 +76,7 @@ def extents(cfg):
 def test_every_target_lies_inside_its_buffer(shape, xe):
     if xe != "fp32" and shape == "72 rows":
         pytest.skip("the 16-bit X-engine takes 64 rows")
-    acc, acc_stored, res, res_stored, acc_read, lost, _, _ = out = extents(SHAPES[shape](xe))
+    acc, acc_stored, res, res_stored, acc_read, lost, *_ = out = extents(SHAPES[shape](xe))
     print(shape, xe, out)
     assert acc_stored <= acc and acc_read <= acc, (acc_stored, acc_read, acc)
     assert 0 < res_stored <= res
@@ -92,6 +92,35 @@ def test_parts_of_a_run_keep_their_length(xe, least, ffts, interval, chunk, long
     cfg = cf.standard_config(4, 2, [4800.0], 32.0, 128, subint_ns=ffts * 4000, xengine=xe, seed=58, chunk_ffts=chunk)
     if interval:
         with_phase_centres(cfg, P=2, interval_ffts=interval, threads=3)
-    *_, run, parts = extents(cfg)
+    *_, run, parts, _ = extents(cfg)
     assert run == longest
     assert 1 <= parts <= max(1, longest // least)
+
+
+MIB = 1 << 20
+
+
+@pytest.mark.parametrize("xe", ["fp32", "fp16"])
+@pytest.mark.parametrize("stations,npol,nfreq,nchan,avg,centres", [
+    (33, 1, 8, 16384, 1, 1), (17, 2, 4, 16384, 1, 1), (33, 1, 8, 16384, 4, 1), (32, 2, 8, 8192, 4, 1), (16, 2, 8, 4096, 1, 3),
+    (4, 1, 1, 256, 1, 1), (32, 1, 2, 256, 1, 1), (10, 2, 8, 1024, 1, 1)])
+def test_accumulators_are_held_once(xe, stations, npol, nfreq, nchan, avg, centres):
+    """The device memory of a context: the chunk's spectra, one set of sums (FP32: a value per
+    product; 16-bit: 8 KiB per channel and pair of row tiles) and no more than 200 MiB beside them,
+    which holds the parts of a split sum (at most 128 MiB), the products on their way to averaging or
+    phase centres (64 MiB, or one freq's) and tables, whatever the job's size."""
+    B = 480
+    cfg = cf.standard_config(stations, npol, [4800.0 + 70.0 * k for k in range(nfreq)], 32.0, nchan,
+                             subint_ns=B * nchan * 1000 // 32, xengine=xe, seed=59, chunk_ffts=64)
+    if avg > 1:
+        averaged(cfg, avg)
+    if centres > 1:
+        with_phase_centres(cfg, P=centres, interval_ffts=40, threads=3)
+    dev, crl, slot = footprint(cfg)
+    n = stations * npol
+    tiles = (n + 31) // 32
+    spectra = nfreq * nchan * 64 * (8 * n if xe == "fp32" else 4 * 32 * tiles)
+    sums = nfreq * nchan * (8 * n * (n + 1) // 2 if xe == "fp32" else 8192 * (tiles * (tiles + 1) // 2))
+    fourstep = 1024 * 2 * nchan * 8 if nchan > 4096 else 0      # the four-step F-engine's rows
+    print(f"{(dev - spectra - sums) / MIB:.1f} MiB beside spectra and sums; slots {slot / MIB:.1f}, results {8 * crl / MIB:.1f}")
+    assert dev <= spectra + sums + 200 * MIB + fourstep
