@@ -191,11 +191,13 @@ struct fxg_ctx {
   DevXGroup* d_groups = nullptr;
   // raw accumulator tiles of either X-engine and their reduction to product accumulators
   float* d_vacc = nullptr;
+  long long vacc_len = 0;
   std::vector<XRGroup> xr_groups;
   std::vector<long long> xr_pairs;
   XRGroup* d_xr_groups = nullptr;
   long long* d_xr_pairs = nullptr;
   int xr_maxC = 0, xr_maxtp = 0;
+  bool fin_sums = false;           // the accumulation reads the sums itself: no reduction
   struct XRBatch { int g0, ng, f0, nf; };   // groups and the accumulation entries that read them
   std::vector<XRBatch> xr_batches;
   float* d_xscale = nullptr;
@@ -1203,6 +1205,42 @@ long long build_xplain(fxg_ctx* ctx) {
   return off;
 }
 
+// Short uv-shift intervals of small arrays: the accumulation reads the sums of the 16-bit X-engine
+// itself and the reduction is left out, where the sums are not split and the products have few
+// values.  50 intervals of 40 FFTs, two phase centres, without and with the reduction: 4 stations dual
+// pol of 256 channels (10K values) 1.54 and 1.77 ms, 16 of 256 (139K) 1.81 and 2.01, 16 of 512 (279K)
+// 2.71 and 2.76, 16 of 1024 (557K) 2.68 both, 4 x 1024 of 10 (901K) 3.29 and 3.11 (one launch less, but
+// a line of the sums read per value and component).
+void sums_read_directly(fxg_ctx* ctx, const std::vector<float>& xs) {
+  long long values = 0;
+  for (const auto& e : ctx->finp) values += (long long)e.nout * e.avg;
+  ctx->fin_sums = ctx->nphase > 1 && values <= 3LL << 17;
+  for (const auto& X : ctx->xr_groups) ctx->fin_sums = ctx->fin_sums && X.nsplit == 1;
+  if (!ctx->fin_sums) return;
+  struct Place { long long src; int g, i, j; };
+  std::vector<Place> at;
+  for (size_t g = 0; g < ctx->xr_groups.size(); ++g) {
+    const XRGroup& X = ctx->xr_groups[g];
+    for (int k = 0; k < X.n * X.n; ++k) {
+      long long& p = ctx->xr_pairs[X.pair0 + k];
+      if (p >= 0) at.push_back({p, (int)g, k / X.n, k % X.n});
+      p = -1;
+    }
+  }
+  std::sort(at.begin(), at.end(), [](const Place& a, const Place& b) { return a.src < b.src; });
+  for (auto& e : ctx->finp) {
+    const Place& q = *--std::upper_bound(at.begin(), at.end(), e.src, [](long long v, const Place& t) { return v < t.src; });
+    const XRGroup& X = ctx->xr_groups[q.g];
+    const bool turned = q.i / 32 < q.j / 32;          // the lower tile of the pair is the stored one
+    const int i = turned ? q.j : q.i, j = turned ? q.i : q.j, ti = i / 32, tj = j / 32;
+    e.tstep = X.ntile * (X.ntile + 1) / 2 * 2048;
+    e.tile = X.off + (e.src - q.src) * e.tstep + (ti * (ti + 1) / 2 + tj) * 2048LL + fxg_mfma_idx(i & 31, j & 31);
+    const float inv = 1.0f / (xs[X.scale_off + i] * xs[X.scale_off + j]);
+    e.sre = inv;
+    e.sim = i == j ? 0.0f : turned ? -inv : inv;
+  }
+}
+
 // Places the product accumulators that are left: those of the per-product kernel, which live through a
 // subint, and then the reduction's, which only pass from it to the accumulation.  The groups go through
 // the latter in batches of at most 64 MiB (or one group), so that jobs whose products are averaged or
@@ -1244,6 +1282,10 @@ void place_accumulators(fxg_ctx* ctx) {
   if (ctx->xr_batches.empty()) ctx->xr_batches.push_back({0, 0, 0, 0});
   std::sort(slots.begin(), slots.end(), [](const Slot& a, const Slot& b) { return a.from < b.from; });
   std::vector<std::vector<FinProd>> fin(ctx->xr_batches.size());
+  if (ctx->fin_sums) {
+    ctx->xr_batches.assign(1, {0, 0, 0, (int)ctx->finp.size()});
+    return;
+  }
   for (FinProd e : ctx->finp) {                    // every entry reads a product that was made above
     const Slot& s = *--std::upper_bound(slots.begin(), slots.end(), e.src, [](long long v, const Slot& t) { return v < t.from; });
     e.src += s.to - s.from;
@@ -1260,6 +1302,7 @@ void place_accumulators(fxg_ctx* ctx) {
 int build_engines(fxg_ctx* ctx, int chunk_req) {
   const int nds = ctx->nds, nb = ctx->nbl;
   const bool mfma = ctx->xengine != FXG_X_FP32;
+  std::vector<float> xs;                           // 16-bit: scale of each group's rows
   // ---- MFMA groups: one per recorded freq table entry, rows = station bands ----
   if (mfma) {
     // freqs that meet in USB x LSB products share a group (one contraction over the rows of
@@ -1377,11 +1420,12 @@ int build_engines(fxg_ctx* ctx, int chunk_req) {
     ctx->xscale_len = soff;
     if (int rc_ = dev_malloc(ctx, (void**)&ctx->d_spec16, sizeof(uint32_t) * std::max<long long>(off, 4))) return rc_;
     if (int rc_ = dev_zero(ctx, ctx->d_spec16, sizeof(uint32_t) * std::max<long long>(off, 4))) return rc_;
+    ctx->vacc_len = aoff;
     if (int rc_ = dev_malloc(ctx, (void**)&ctx->d_vacc, sizeof(float) * std::max<long long>(aoff, 4))) return rc_;
     // nominal per-input scale 1/sqrt(L <x^2>) of the input's sample levels, which keeps the
     // 16-bit spectra near unit magnitude; the accumulation divides it out again
     const double p_hi = 0.5 * std::erfc(0.95 / std::sqrt(2.0));
-    std::vector<float> xs((size_t)std::max<long long>(soff, 1), 0.0f);
+    xs.assign((size_t)std::max<long long>(soff, 1), 0.0f);
     for (size_t g = 0; g < ctx->groups.size(); ++g)
       for (size_t r = 0; r < ctx->group_rows[g].size(); ++r) {
         const int d = ctx->group_rows[g][r].first;
@@ -1609,6 +1653,7 @@ int build_engines(fxg_ctx* ctx, int chunk_req) {
     ctx->xr_maxC = std::max(ctx->xr_maxC, X.C);
     ctx->xr_maxtp = std::max(ctx->xr_maxtp, X.ntile * (X.ntile + 1) / 2);
   }
+  if (mfma) sums_read_directly(ctx, xs);
   place_accumulators(ctx);
   if (int rc = dev_malloc(ctx, (void**)&ctx->d_xacc, (long long)sizeof(float2) * std::max<long long>(ctx->xacc_len, 2))) return rc;
   if (!ctx->prods_rest.empty())
@@ -2113,7 +2158,7 @@ int run_subint(fxg_ctx* ctx, const int32_t offsets[3], const uint8_t* const* d_d
     for (const auto& b : ctx->xr_batches) {
       ra.groups = ctx->d_xr_groups + b.g0;
       if (fxg_launch_xreduce(ra, mfma, b.ng, ctx->xr_maxC, ctx->xr_maxtp, st) ||
-          fxg_launch_fin(ctx->d_finp + b.f0, b.nf, ctx->maxoutp, ctx->d_xacc, d_results, u, st))
+          fxg_launch_fin(ctx->d_finp + b.f0, b.nf, ctx->maxoutp, ctx->d_xacc, ctx->fin_sums ? ctx->d_vacc : nullptr, d_results, u, st))
         return fail(ctx, FXG_E_HIP, "accumulate launch");
     }
     return FXG_OK;
@@ -3418,7 +3463,7 @@ int fxg_autotune_report(const fxg_ctx* ctx, char* buf, int32_t len) {
 // The extents of the X-engine's stores, for tests of the tables of any context (a host-only one
 // included): out = {entries of the product accumulators, end of the furthest store into them,
 // entries of the results, end of the furthest store into them, end of the furthest read of the
-// product accumulators, reads of entries that nothing stores, FFTs of the longest run of an
+// product accumulators, reads of entries that nothing stores (or outside the sums), FFTs of the longest run of an
 // X-engine loop, most parts that one is split into, batches of the accumulation}.  Entries are
 // complex values.
 int fxg_x_extents(const fxg_ctx* ctx, int64_t out[9]) {
@@ -3444,7 +3489,12 @@ int fxg_x_extents(const fxg_ctx* ctx, int64_t out[9]) {
       const FinProd& e = ctx->finp[f];
       const int np = ctx->nphase > 1 && e.bl >= 0 ? ctx->nphase : 1;
       rend = std::max(rend, (long long)e.dst + (long long)(np - 1) * e.pcstride + e.nout);
-      const long long r1 = e.src + (long long)e.nout * e.avg;
+      const long long n = (long long)e.nout * e.avg;
+      if (ctx->fin_sums) {                              // reads the sums themselves
+        if (e.tile < 0 || e.tile + (n - 1) * e.tstep + 1024 >= ctx->vacc_len) ++lost;
+        continue;
+      }
+      const long long r1 = e.src + n;
       read = std::max(read, r1);
       auto it = std::upper_bound(st.begin(), st.end(), std::pair<long long, long long>(e.src, 1LL << 62));
       if (it == st.begin() || r1 > (--it)->second) ++lost;

@@ -310,6 +310,11 @@ struct FinProd {
   int bl;                 // baseline of a cross product (-1: autocorrelation, not shifted)
   int fq;                 // freq of the product (uv-shift rotation constants)
   int pcstride;           // cf32 offset between the phase-centre blocks
+  // where the accumulation reads the 16-bit X-engine's sums itself: the value of channel c is
+  // (part[tile + c tstep] sre, part[tile + 1024 + c tstep] sim)
+  long long tile;
+  int tstep;
+  float sre, sim;
 };
 
 struct FinWeight {
@@ -343,7 +348,9 @@ void fxg_fmat_tables(uint32_t* out);
 int fxg_launch_fmat(const FengineArgs& a, int nds, int ncu, int nfreqs, const uint32_t* tables, hipStream_t st);
 int fxg_launch_xplain(const XPlainArgs& a, int nprod, int maxchan, hipStream_t st);
 int fxg_launch_xmfma(const XMfmaArgs& a, int ngroup_launch, int group0, const DevXGroup& g, hipStream_t st);
-int fxg_launch_fin(const FinProd* e, int n, int maxout, const float2* acc, float2* res, const UvArgs& uv, hipStream_t st);
+int fxg_mfma_idx(int i, int j);              // element (i, j) of a stored 32 x 32 tile
+int fxg_launch_fin(const FinProd* e, int n, int maxout, const float2* acc, const float* part, float2* res, const UvArgs& uv,
+                   hipStream_t st);   // part: read the sums from there (FinProd::tile); null: the products from acc
 int fxg_launch_add_at(const int* idx, const float* val, int n, float* resf, hipStream_t st);
 int fxg_launch_fin_weights(const FinWeight* e, int n, const float* w, int B, float* resf, hipStream_t st);
 int fxg_launch_zero(void* p, long long bytes, hipStream_t st);

@@ -418,7 +418,7 @@ __global__ void __launch_bounds__((XTile<NTILE, CT_>::NTH)) k_xmac_mfma(XMfmaArg
 
 // Register r of lane l of a 32x32 MFMA accumulator holds element
 //   (i, j) = (8*(r/4) + 4*(l/32) + r%4, l%32).
-__device__ __forceinline__ int mfma_idx(int i, int j) {
+__host__ __device__ __forceinline__ int mfma_idx(int i, int j) {
   const int r = (i >> 3) * 4 + (i & 3);
   const int l = ((i >> 2) & 1) * 32 + j;
   return r * 64 + l;
@@ -566,8 +566,17 @@ __device__ __forceinline__ float2 uv_rotate(float2 v, double dd, const UvFreq& q
   return make_float2(r.x * c2 - r.y * s2, r.x * s2 + r.y * c2);
 }
 
-__global__ void k_fin(const FinProd* e, const float2* acc, float2* res, UvArgs uv) {
+// One workgroup row per product.  SUMS: without the reduction's pass over LDS and memory, straight
+// from the 16-bit X-engine's sums (a value per 128-byte line and component): a launch less, which is
+// what counts in short uv-shift intervals of small arrays (see sums_read_directly).
+template <bool SUMS>
+__global__ void k_fin(const FinProd* e, const float2* acc, const float* part, float2* res, UvArgs uv) {
   const FinProd f = e[blockIdx.y];
+  auto value = [&](int ch) {
+    if (!SUMS) return acc[f.src + ch];
+    const float* p = part + f.tile + (long long)ch * f.tstep;
+    return make_float2(p[0] * f.sre, p[1024] * f.sim);
+  };
   const int co = blockIdx.x * blockDim.x + threadIdx.x;
   if (co >= f.nout) return;
   if (uv.P > 1 && f.bl >= 0) {                    // rotated into every phase centre's block
@@ -578,7 +587,7 @@ __global__ void k_fin(const FinProd* e, const float2* acc, float2* res, UvArgs u
       float2 s = make_float2(0.f, 0.f);
       for (int k = 0; k < f.avg; ++k) {
         const int ch = co * f.avg + k;
-        float2 v = acc[f.src + ch];
+        float2 v = value(ch);
         if (turn) v = uv_rotate(v, dd, q, ch);
         s.x += v.x; s.y += v.y;
       }
@@ -590,7 +599,7 @@ __global__ void k_fin(const FinProd* e, const float2* acc, float2* res, UvArgs u
   }
   float2 s = make_float2(0.f, 0.f);
   for (int k = 0; k < f.avg; ++k) {
-    const float2 v = acc[f.src + (long long)co * f.avg + k];
+    const float2 v = value(co * f.avg + k);
     s.x += v.x; s.y += v.y;
   }
   if (f.avg > 1) { s.x /= (float)f.avg; s.y /= (float)f.avg; }
@@ -707,12 +716,16 @@ int fxg_launch_xmfma(const XMfmaArgs& a, int ngroup_launch, int group0, const De
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
 
-int fxg_launch_fin(const FinProd* e, int n, int maxout, const float2* acc, float2* res, const UvArgs& uv,
-                         hipStream_t st) {
+int fxg_launch_fin(const FinProd* e, int n, int maxout, const float2* acc, const float* part, float2* res, const UvArgs& uv,
+                   hipStream_t st) {
   if (n == 0) return 0;
-  hipLaunchKernelGGL(k_fin, dim3((maxout + 255) / 256, n), dim3(256), 0, st, e, acc, res, uv);
+  const dim3 grid((maxout + 255) / 256, n);
+  if (part) hipLaunchKernelGGL(k_fin<true>, grid, dim3(256), 0, st, e, acc, part, res, uv);
+  else hipLaunchKernelGGL(k_fin<false>, grid, dim3(256), 0, st, e, acc, part, res, uv);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
+
+int fxg_mfma_idx(int i, int j) { return mfma_idx(i, j); }
 
 int fxg_launch_add_at(const int* idx, const float* val, int n, float* resf, hipStream_t st) {
   if (n == 0) return 0;

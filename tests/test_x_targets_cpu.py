@@ -41,7 +41,15 @@ def averaged(cfg, n=4):
     return cfg
 
 
+def large_phase_centres(xe):
+    """More values than the accumulation reads without the reduction, in two freqs of two row tiles."""
+    cfg = cf.standard_config(20, 2, [4800.0, 4840.0], 32.0, 512, subint_ns=24 * 16000, xengine=xe, seed=60,
+                             max_delay_us=50.0)
+    return with_phase_centres(cfg, P=2, interval_ffts=8, threads=2)
+
+
 SHAPES = {
+    "phase centres, 40 rows": large_phase_centres,
     "parallel hands": parallel_hands,
     "parallel hands, no cross autos": lambda xe: parallel_hands(xe, write_cross_autocorrs=False),
     "parallel hands averaged": lambda xe: averaged(parallel_hands(xe)),
