@@ -716,7 +716,7 @@ def main():
         usamp = samples_per_subint(tcfg)
         forms = {}
         usteps = 5
-        for name, mode in (("per_length", 0), ("persistent", 2)):
+        for name, mode in (("automatic", 0), ("persistent", 2)):
             ucfg = uneven_config("fp16", fengine_mode=mode)
             print(f"[bench] uneven bands ({name} F-engine launch), 1 warmup + {usteps} steps", file=sys.stderr, flush=True)
             u = time_path(ucfg, usteps, 1, torch, dev, offsets)

@@ -335,7 +335,7 @@ int fxg_launch_fbig(const FengineArgs& a, int L, int iscomplex, int nds, int wgx
                     const float2* twL, hipStream_t st);
 size_t fxg_fbig_lds(int ntb, int phcap);
 
-// Register F-engine (fxg_freg.hip): long FFTs of real 2-bit samples.
+// Register F-engine (fxg_freg.hip): long FFTs of real 2-bit and complex 8-bit samples.
 bool fxg_freg_takes(int L, int cplx, int nbits, int order, int S, int phcap);
 const std::vector<float2>& fxg_freg_tables(int L);
 int fxg_launch_freg(const FengineArgs& a, int L, int cplx, int nds, int ncu, const float2* tw, hipStream_t st);

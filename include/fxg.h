@@ -202,7 +202,9 @@ int fxg_process_subint(fxg_ctx* ctx, const int32_t offsets[3], const uint8_t* co
 /* Same, with the data already resident in device memory (d_data[ds]) and the results
  * written to device memory (d_results, coreresultlength cf32).  Work is enqueued on
  * `stream` (a hipStream_t, may be null for the context's own stream) and is complete when
- * the stream is.  Control words are read from host memory before the call returns. */
+ * the stream is.  Control words are read from host memory before the call returns.  Frames are read
+ * in words of up to 8 bytes: buffers at other than 8-byte boundaries rely on the hardware's unaligned
+ * loads. */
 int fxg_process_subint_device(fxg_ctx* ctx, const int32_t offsets[3],
                               const uint8_t* const* d_data, const int32_t* nbytes,
                               const int32_t* const* control, float* d_results, void* stream);
@@ -228,7 +230,9 @@ int fxg_get_data_weights(const fxg_ctx* ctx, int32_t ds, float* out /* [blockspe
  * (numblocks s2 / s1^2 - 1) numblocks/(numblocks-1) - 1, numblocks = blockspersend, summed
  * over groups of C/maxchannels channels (and divided by the group size) when maxchannels < C;
  * *nout = the values written (0 when the band had no data, where the reference sends no
- * record). */
+ * record).  Where the spectra are 16-bit and the launch form is automatic, a subint with the sums on
+ * uses the per-length F-engine kernels: its visibilities differ by the rounding of the spectra from
+ * those without, and 2048-point and longer FFTs take as long as with FXG_F_PER_LENGTH. */
 int fxg_set_kurtosis(fxg_ctx* ctx, int32_t enable);
 /* The STA autocorrelation record data of a recorded band (Core::averageAndSendAutocorrs,
  * core.cpp:1166-1258) from a slot's results (host memory): the parallel autocorrelation's real
