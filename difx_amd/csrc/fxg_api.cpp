@@ -1233,8 +1233,9 @@ void sums_read_directly(fxg_ctx* ctx, const std::vector<float>& xs) {
     const XRGroup& X = ctx->xr_groups[q.g];
     const bool turned = q.i / 32 < q.j / 32;          // the lower tile of the pair is the stored one
     const int i = turned ? q.j : q.i, j = turned ? q.i : q.j, ti = i / 32, tj = j / 32;
-    e.tstep = X.ntile * (X.ntile + 1) / 2 * 2048;
-    e.tile = X.off + (e.src - q.src) * e.tstep + (ti * (ti + 1) / 2 + tj) * 2048LL + fxg_mfma_idx(i & 31, j & 31);
+    e.tstep = xh_floats(X.n);
+    e.im = xh_len(X.n, ti, tj);
+    e.tile = X.off + (e.src - q.src) * e.tstep + xh_tile(X.n, ti * (ti + 1) / 2 + tj) + (i & 31) * xp_rows(X.n, tj) + (j & 31);
     const float inv = 1.0f / (xs[X.scale_off + i] * xs[X.scale_off + j]);
     e.sre = inv;
     e.sim = i == j ? 0.0f : turned ? -inv : inv;
@@ -1410,7 +1411,7 @@ int build_engines(fxg_ctx* ctx, int chunk_req) {
       g.spec_off = off;
       g.rowstride = cap * g.C + 32;       // one 128-byte line of padding per row
       off += (long long)g.ntile * 32 * g.rowstride;
-      g.split_stride = (long long)g.C * (g.ntile * (g.ntile + 1) / 2) * 2 * 1024;
+      g.split_stride = (long long)g.C * xh_floats(g.nin);
       g.acc_off = aoff;
       aoff += g.nsplit * g.split_stride;
       g.scale_off = soff;
@@ -3491,7 +3492,7 @@ int fxg_x_extents(const fxg_ctx* ctx, int64_t out[9]) {
       rend = std::max(rend, (long long)e.dst + (long long)(np - 1) * e.pcstride + e.nout);
       const long long n = (long long)e.nout * e.avg;
       if (ctx->fin_sums) {                              // reads the sums themselves
-        if (e.tile < 0 || e.tile + (n - 1) * e.tstep + 1024 >= ctx->vacc_len) ++lost;
+        if (e.tile < 0 || e.tile + (n - 1) * e.tstep + e.im >= ctx->vacc_len) ++lost;
         continue;
       }
       const long long r1 = e.src + n;

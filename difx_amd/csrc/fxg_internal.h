@@ -230,6 +230,13 @@ __host__ __device__ constexpr int xp_tile(int n, int ti, int tj) {
   return n <= 32 ? 0 : ti == 0 ? tj * 1024 : 32 * n + tj * 32 * (n - 32);
 }
 __host__ __device__ constexpr int xp_floats(int n) { return (n * n + 3) & ~3; }
+// The same of the 16-bit X-engine: floats of one part of tile (ti, tj), tj <= ti, the place of tile pair
+// ti (ti + 1) / 2 + tj, and a channel's floats in all.
+__host__ __device__ constexpr int xh_len(int n, int ti, int tj) { return (xp_rows(n, ti) * xp_rows(n, tj) + 3) & ~3; }
+__host__ __device__ constexpr int xh_tile(int n, int pair) { return pair == 0 ? 0 : pair == 1 ? 2048 : 2048 + 64 * (n - 32); }
+__host__ __device__ constexpr int xh_floats(int n) {
+  return n <= 32 ? 2 * xh_len(n, 0, 0) : xh_tile(n, 2) + 2 * xh_len(n, 1, 1);
+}
 struct XPGroup {
   int nrows, C, row0;       // rows[row0 + i]: cf32 offset of (band, FFT 0, window start)
   int stride;               // cf32 entries between consecutive FFTs, the same for every row
@@ -253,7 +260,8 @@ struct XPMatArgs {
 // Raw accumulator tiles of either X-engine into per-product rows of channels: the splits over
 // FFTs are summed in order and product (i, j) of a group goes, by its pair table entry p, to
 // acc[p + c] (p >= 0), straight to the results, res[-2 - p + c] (p <= -2), or nowhere (-1).
-// FP32: the matrix S per channel (xp_floats); 16-bit: (re, im) 32 x 32 tiles of the lower tile pairs.
+// FP32: the matrix S per channel (xp_floats); 16-bit: V's lower tiles per channel, real parts and
+// then imaginary parts of each (xh_floats).
 struct XRGroup {
   int n, C, ntile, pad;
   long long off;            // float offset of split 0, channel 0
@@ -311,9 +319,9 @@ struct FinProd {
   int fq;                 // freq of the product (uv-shift rotation constants)
   int pcstride;           // cf32 offset between the phase-centre blocks
   // where the accumulation reads the 16-bit X-engine's sums itself: the value of channel c is
-  // (part[tile + c tstep] sre, part[tile + 1024 + c tstep] sim)
+  // (part[tile + c tstep] sre, part[tile + im + c tstep] sim)
   long long tile;
-  int tstep;
+  int tstep, im;
   float sre, sim;
 };
 
@@ -348,7 +356,6 @@ void fxg_fmat_tables(uint32_t* out);
 int fxg_launch_fmat(const FengineArgs& a, int nds, int ncu, int nfreqs, const uint32_t* tables, hipStream_t st);
 int fxg_launch_xplain(const XPlainArgs& a, int nprod, int maxchan, hipStream_t st);
 int fxg_launch_xmfma(const XMfmaArgs& a, int ngroup_launch, int group0, const DevXGroup& g, hipStream_t st);
-int fxg_mfma_idx(int i, int j);              // element (i, j) of a stored 32 x 32 tile
 int fxg_launch_fin(const FinProd* e, int n, int maxout, const float2* acc, const float* part, float2* res, const UvArgs& uv,
                    hipStream_t st);   // part: read the sums from there (FinProd::tile); null: the products from acc
 int fxg_launch_add_at(const int* idx, const float* val, int n, float* resf, hipStream_t st);

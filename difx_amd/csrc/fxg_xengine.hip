@@ -312,22 +312,39 @@ __global__ void __launch_bounds__((XTile<NTILE, CT_>::NTH)) k_xmac_mfma(XMfmaArg
     (&lds_raw[0][0])[i] = make_uint4(0u, 0u, 0u, 0u);
 
   floatx16 accr[CPW][NPAIR], acci[CPW][NPAIR];
-  float* acc0 = a.acc + g.acc_off + blockIdx.z * g.split_stride;
+  // the sums of channel c, tile pair p: the group's rows only; register r of a lane is element
+  // (8 (r / 4) + 4 half + r % 4, row) of the tile
+  const int cs = xh_floats(g.nin);
+  float* acc0 = a.acc + g.acc_off + blockIdx.z * g.split_stride + (long long)(c0 + wave * CPW) * cs;
+  auto sums = [&](auto&& f) {
+    int p = 0;
 #pragma unroll
-  for (int cw = 0; cw < CPW; ++cw) {
-    const int c = c0 + wave * CPW + cw;
-    const float* accp = acc0 + (long long)c * NPAIR * 2 * 1024;
+    for (int ti = 0; ti < NTILE; ++ti)
 #pragma unroll
-    for (int p = 0; p < NPAIR; ++p) {
-      const float* pr = accp + (p * 2 + 0) * 1024 + lane;    // immediate offsets r * 256 bytes
-      const float* pi = accp + (p * 2 + 1) * 1024 + lane;
+      for (int tj = 0; tj <= ti; ++tj, ++p) {
+        const int h = xp_rows(g.nin, ti), w = xp_rows(g.nin, tj);
+        float* pt = acc0 + xh_tile(g.nin, p) + row;
+        const int im = xh_len(g.nin, ti, tj);
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        accr[cw][p][r] = a.first ? 0.0f : pr[r * 64];
-        acci[cw][p][r] = a.first ? 0.0f : pi[r * 64];
+        for (int r = 0; r < 16; ++r) {
+          const int i = 8 * (r >> 2) + 4 * half + (r & 3);
+          if (i >= h || row >= w) continue;
+#pragma unroll
+          for (int cw = 0; cw < CPW; ++cw) f(pt + cw * cs + i * w, im, cw, p, r);
+        }
       }
-    }
-  }
+  };
+#pragma unroll
+  for (int cw = 0; cw < CPW; ++cw)
+#pragma unroll
+    for (int p = 0; p < NPAIR; ++p)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) accr[cw][p][r] = acci[cw][p][r] = 0.0f;
+  if (!a.first)
+    sums([&](const float* v, int im, int cw, int p, int r) {
+      accr[cw][p][r] = v[0];
+      acci[cw][p][r] = v[im];
+    });
 
   // chunk q of a k-step: row r = q / QPR, FFT t = (q % QPR) / (CT/4), channel quad
   // h = q % (CT/4).  The loads are unconditional (a chunk past the group's inputs re-reads
@@ -399,29 +416,10 @@ __global__ void __launch_bounds__((XTile<NTILE, CT_>::NTH)) k_xmac_mfma(XMfmaArg
     __syncthreads();
   }
 
-#pragma unroll
-  for (int cw = 0; cw < CPW; ++cw) {
-    const int c = c0 + wave * CPW + cw;
-    float* accp = acc0 + (long long)c * NPAIR * 2 * 1024;
-#pragma unroll
-    for (int p = 0; p < NPAIR; ++p) {
-      float* pr = accp + (p * 2 + 0) * 1024 + lane;
-      float* pi = accp + (p * 2 + 1) * 1024 + lane;
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        pr[r * 64] = accr[cw][p][r];
-        pi[r * 64] = acci[cw][p][r];
-      }
-    }
-  }
-}
-
-// Register r of lane l of a 32x32 MFMA accumulator holds element
-//   (i, j) = (8*(r/4) + 4*(l/32) + r%4, l%32).
-__host__ __device__ __forceinline__ int mfma_idx(int i, int j) {
-  const int r = (i >> 3) * 4 + (i & 3);
-  const int l = ((i >> 2) & 1) * 32 + j;
-  return r * 64 + l;
+  sums([&](float* v, int im, int cw, int p, int r) {
+    v[0] = accr[cw][p][r];
+    v[im] = acci[cw][p][r];
+  });
 }
 
 // The raw accumulator tiles to the products: a workgroup reads a block of tiles of a few
@@ -456,7 +454,7 @@ __device__ __forceinline__ void xr_put(const XReduceArgs& a, long long p, int c,
   else if (p < -1) a.res[-2 - p + c] = v;
 }
 
-// 16-bit X-engine: 16 channels, one pair of row tiles, eight rows (256 floats of each tile).
+// 16-bit X-engine: 16 channels, one pair of row tiles, eight rows (up to 256 floats of each part).
 constexpr int XRH_CH = 16, XRH_CS = 512 + 4;
 __global__ void __launch_bounds__(256) k_xreduce_h(XReduceArgs a) {
   __shared__ float s[XRH_CH * XRH_CS];
@@ -467,8 +465,9 @@ __global__ void __launch_bounds__(256) k_xreduce_h(XReduceArgs a) {
   while (tj > ti) { ++ti; tj -= ti; }
   if (c0 >= g.C || tp >= ntp || ti * 32 + i0 >= g.n) return;
   const int nch = min(XRH_CH, g.C - c0);
-  const long long chf = (long long)ntp * 2048;
-  const float* p = a.part + g.off + c0 * chf + (long long)tp * 2048 + i0 * 32;
+  const long long chf = xh_floats(g.n);
+  const int w = xp_rows(g.n, tj), len = (min(8, xp_rows(g.n, ti) - i0) * w + 3) & ~3;
+  const float* p = a.part + g.off + c0 * chf + xh_tile(g.n, tp) + i0 * w;
   // the places and the rows' scales are on their way while the parts are added: a small call's
   // reduction is a chain of such loads (5.5 us with them in the loop below)
   __shared__ float rs[8 + 32];
@@ -486,7 +485,7 @@ __global__ void __launch_bounds__(256) k_xreduce_h(XReduceArgs a) {
     const int r = threadIdx.x < 8 ? ti * 32 + i0 + (int)threadIdx.x : tj * 32 + (int)threadIdx.x - 8;
     rs[threadIdx.x] = r < g.n ? a.xscale[g.scale_off + r] : 1.0f;
   }
-  xr_gather<2, XRH_CH>(s, p, p + 1024, chf, nch, 256, XRH_CS, g.nsplit, g.split_stride);
+  xr_gather<2, XRH_CH>(s, p, p + xh_len(g.n, ti, tj), chf, nch, len, XRH_CS, g.nsplit, g.split_stride);
   __syncthreads();
   const int ch = threadIdx.x % XRH_CH;
   if (ch >= nch) return;
@@ -496,8 +495,8 @@ __global__ void __launch_bounds__(256) k_xreduce_h(XReduceArgs a) {
     if (pp[n] == -1 && pq[n] == -1) continue;
     const int e = threadIdx.x / XRH_CH + n * (256 / XRH_CH), i = e >> 5, j = e & 31;
     const float inv = 1.0f / (rs[i] * rs[8 + j]);
-    const int k = mfma_idx(i, j);
-    float2 v = make_float2(sc[k] * inv, sc[256 + k] * inv);
+    const int k = i * w + j;
+    float2 v = make_float2(sc[k] * inv, sc[len + k] * inv);
     if (ti == tj && i0 + i == j) v.y = 0.0f;               // x conj(x) is real
     xr_put(a, pp[n], c0 + ch, v);
     xr_put(a, pq[n], c0 + ch, make_float2(v.x, -v.y));
@@ -575,7 +574,7 @@ __global__ void k_fin(const FinProd* e, const float2* acc, const float* part, fl
   auto value = [&](int ch) {
     if (!SUMS) return acc[f.src + ch];
     const float* p = part + f.tile + (long long)ch * f.tstep;
-    return make_float2(p[0] * f.sre, p[1024] * f.sim);
+    return make_float2(p[0] * f.sre, p[f.im] * f.sim);
   };
   const int co = blockIdx.x * blockDim.x + threadIdx.x;
   if (co >= f.nout) return;
@@ -724,8 +723,6 @@ int fxg_launch_fin(const FinProd* e, int n, int maxout, const float2* acc, const
   else hipLaunchKernelGGL(k_fin<false>, grid, dim3(256), 0, st, e, acc, part, res, uv);
   return hipGetLastError() == hipSuccess ? 0 : -1;
 }
-
-int fxg_mfma_idx(int i, int j) { return mfma_idx(i, j); }
 
 int fxg_launch_add_at(const int* idx, const float* val, int n, float* resf, hipStream_t st) {
   if (n == 0) return 0;

@@ -132,3 +132,17 @@ def test_accumulators_are_held_once(xe, stations, npol, nfreq, nchan, avg, centr
     fourstep = 1024 * 2 * nchan * 8 if nchan > 4096 else 0      # the four-step F-engine's rows
     print(f"{(dev - spectra - sums) / MIB:.1f} MiB beside spectra and sums; slots {slot / MIB:.1f}, results {8 * crl / MIB:.1f}")
     assert dev <= spectra + sums + 200 * MIB + fourstep
+
+
+@pytest.mark.parametrize("xe", ["fp32", "fp16"])
+def test_parts_hold_the_rows_of_their_group(xe):
+    """4 stations dual pol x 256 channels, 8000 FFTs: the parts of the split sums take 64 (FP32) or 128
+    values per channel, not whole tiles: no more than 16 MiB beside the spectra, the delay parameters
+    and weights."""
+    cfg = cf.standard_config(4, 2, [4800.0], 32.0, 256, subint_ns=8000 * 8000, xengine=xe, seed=61)
+    *_, parts, _ = extents(cfg)
+    assert parts > 8
+    dev, _, _ = footprint(cfg)
+    spectra = 256 * 8000 * (8 * 8 if xe == "fp32" else 4 * 32)
+    print(f"{parts} parts, {(dev - spectra) / MIB:.1f} MiB beside the spectra")
+    assert dev <= spectra + 16 * MIB
