@@ -1208,9 +1208,9 @@ long long build_xplain(fxg_ctx* ctx) {
 // Short uv-shift intervals of small arrays: the accumulation reads the sums of the 16-bit X-engine
 // itself and the reduction is left out, where the sums are not split and the products have few
 // values.  50 intervals of 40 FFTs, two phase centres, without and with the reduction: 4 stations dual
-// pol of 256 channels (10K values) 1.54 and 1.77 ms, 16 of 256 (139K) 1.81 and 2.01, 16 of 512 (279K)
-// 2.71 and 2.76, 16 of 1024 (557K) 2.68 both, 4 x 1024 of 10 (901K) 3.29 and 3.11 (one launch less, but
-// a line of the sums read per value and component).
+// pol of 256 channels (10K values) 1.42 and 1.63 ms, 16 of 256 (139K) 1.77 and 1.99, 16 of 512 (279K)
+// 2.67 and 2.74; 10 of 2 x 1024 (451K) 2.56 and 2.45, of 4 x 1024 (901K) 3.24 and 2.88 (one launch less,
+// but a line of the sums read for a few of its values).
 void sums_read_directly(fxg_ctx* ctx, const std::vector<float>& xs) {
   long long values = 0;
   for (const auto& e : ctx->finp) values += (long long)e.nout * e.avg;
@@ -1398,7 +1398,8 @@ int build_engines(fxg_ctx* ctx, int chunk_req) {
   if (mfma) {
     // Split each launch's FFT loop (groups of one shape run together) so that it has two
     // workgroups per CU: 32 stations x 256 channels (64 channel tiles) 2000 -> 1280 us per subint;
-    // four or eight per CU cost more in accumulator traffic than they gain (1316, 1395 us).
+    // four or eight per CU cost more in accumulator traffic than they gain (1316, 1395 us; all three
+    // with the sums in whole tiles, 1190 us for two per CU since).
     for (size_t g0 = 0, g1; g0 < ctx->groups.size(); g0 = g1) {
       const DevXGroup& G = ctx->groups[g0];
       for (g1 = g0; g1 < ctx->groups.size() && ctx->groups[g1].ntile == G.ntile && ctx->groups[g1].C == G.C; ++g1) {}

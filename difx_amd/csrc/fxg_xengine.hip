@@ -425,7 +425,7 @@ __global__ void __launch_bounds__((XTile<NTILE, CT_>::NTH)) k_xmac_mfma(XMfmaArg
 // The raw accumulator tiles to the products: a workgroup reads a block of tiles of a few
 // channels of one group into LDS, whole lines at a time, summing the splits in order, and then
 // writes one value per thread with the channel fastest, so each product gets 64- or 128-byte
-// runs (read in place, the 4-byte values of one product are 1 to 16 KB apart).  A product whose
+// runs (read in place, the 4-byte values of one product are a channel's sums, up to 24 KB, apart).  A product whose
 // channels go to the results as they are is written there, the others to their accumulators.
 template <int NPL, int CH>
 __device__ __forceinline__ void xr_gather(float* s, const float* p0, const float* p1, long long chf, int nch, int len,
@@ -566,7 +566,7 @@ __device__ __forceinline__ float2 uv_rotate(float2 v, double dd, const UvFreq& q
 }
 
 // One workgroup row per product.  SUMS: without the reduction's pass over LDS and memory, straight
-// from the 16-bit X-engine's sums (a value per 128-byte line and component): a launch less, which is
+// from the 16-bit X-engine's sums (a row of them per channel): a launch less, which is
 // what counts in short uv-shift intervals of small arrays (see sums_read_directly).
 template <bool SUMS>
 __global__ void k_fin(const FinProd* e, const float2* acc, const float* part, float2* res, UvArgs uv) {
