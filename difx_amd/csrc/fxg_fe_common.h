@@ -5,6 +5,7 @@
 #include "../../include/fxg.h"
 #include <hip/hip_fp16.h>
 #include <hip/hip_bf16.h>
+#include <mutex>
 
 namespace {
 
@@ -829,10 +830,15 @@ __device__ void fe_range(const FengineArgs& args, const float2* __restrict__ twi
   }
 }
 
-// Raise a kernel's dynamic-LDS limit once where a launch needs more than the default.
+// Raise a kernel's dynamic-LDS limit once where a launch needs more than the default.  One thread at
+// a time: contexts of other threads launch the same kernels with table sizes of their own, and the
+// limit must not fall back to a smaller one's.
 template <typename K>
 static int raise_lds(K kern, size_t lds, size_t* raised) {
-  if (lds > 65536 && lds > *raised) {
+  if (lds <= 65536) return 0;
+  static std::mutex mu;
+  std::lock_guard<std::mutex> lk(mu);
+  if (lds > *raised) {
     if (hipFuncSetAttribute((const void*)kern, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds) != hipSuccess)
       return -1;
     *raised = lds;
